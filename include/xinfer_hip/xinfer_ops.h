@@ -29,7 +29,8 @@
  * the code object loader places with the library's kernels: 32 slots of
  * 4 MiB + 16 KiB (128.5 MiB) on every device the library runs on, one
  * owned by each stream that calls until xinfer_stream_release gives it
- * back; with every slot owned a call plans without the cross-block split
+ * back; the first 8 also hold 64 MiB each (512 MiB) for the partial sums of
+ * the prefill GEMM (M > 16); with every slot owned a call plans without the cross-block split
  * (correct, slower).  Calls on different streams may therefore overlap.  A
  * graph holds the slot of the stream it was captured on: replays of graphs
  * captured on one stream must not overlap each other or that stream's work
@@ -82,11 +83,11 @@ const char* xinfer_version(void);
  * M <= 16 runs the bandwidth-bound decode kernels (VALU GEMV at M = 1-2,
  * MFMA small-batch kernel at M = 2-16); larger M (chunked prefill) runs the
  * MFMA GEMM, as the reference routes both through this one call
- * (src/targets/qwen3_8/forward.cpp:284-287).  Dequantisation: the decode
- * kernels (M <= 16) and fp32 outputs at any M multiply the exact integer q
- * by the FP32 group scale, as the reference does; the fp16-output prefill
- * GEMM (M > 16) feeds the matrix cores B = fp16(q*s), rounded once per
- * weight (relative error <= 2^-11, inside the fp16 output's rounding).
+ * (src/targets/qwen3_8/forward.cpp:284-287).  Dequantisation: every kernel
+ * multiplies the exact integer q by the FP32 group scale, as the reference
+ * does, but for one: fp16 outputs of launches that fill the chip with 256-row
+ * blocks feed the matrix cores B = fp16(q*s), rounded once per weight
+ * (relative error <= 2^-11, inside the fp16 output's rounding).
  * ------------------------------------------------------------------------- */
 
 /* Replaces `sycl::event linear_int4(sycl::queue&, sycl::half* Y,

@@ -41,3 +41,18 @@ def test_pair_split(tmp_path):
     run = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     print(run.stdout)
     assert run.returncode == 0, run.stdout[-2000:]
+
+
+@pytest.mark.skipif(_hipcc() is None, reason="hipcc not available")
+def test_prefill_gemm_split(tmp_path):
+    """The prefill GEMM's work split: runs, pieces and the second launch that
+    adds them, over 20000 random calls."""
+    exe = str(tmp_path / "sk_plan_check")
+    build = subprocess.run([_hipcc(), "-O1", "-std=c++17", "--offload-arch=gfx950",
+                            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                            os.path.join(HERE, "sk_plan_check.hip"), "-o", exe],
+                           capture_output=True, text=True, timeout=900)
+    assert build.returncode == 0, build.stderr[-2000:]
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    print(run.stdout)
+    assert run.returncode == 0, run.stdout[-2000:]

@@ -846,9 +846,8 @@ int mb_argmax_plan(int64_t M, int64_t N, int64_t K, int* nparts);
 int mb_max_m();  // largest M the small-batch kernel takes (then the GEMM)
 int mb_argmax(hipStream_t st, float* logits, const void* X, const uint8_t* W, const void* S,
               int64_t M, int64_t N, int64_t K, ArgCand* parts, int* nparts, int* rc);
-int gemm_int4_f16(hipStream_t st, void* Y, bool y_f32, const void* X, const uint8_t* W,
-                  const uint16_t* S, const uint8_t* W2, const uint16_t* S2, const float* bias,
-                  int64_t M, int64_t N, int64_t K, bool residual = false);
+int prefill_gemm(hipStream_t st, const xinfer_fused_desc* descs, int nd, const uint8_t* W2, const uint16_t* S2,
+                 const void* X, bool y_f32, int64_t M, int64_t K, bool residual);  // gemm_sk_int4.hip
 }
 
 namespace {
@@ -871,9 +870,10 @@ int linear_f16_impl(void* stream, void* Y, bool y_f32, const void* X, const uint
         if (!pairm_linear(st, &one, 1, X, y_f32, M, K, residual, &mrc)) return mrc;
         if (!mb_linear(st, &one, 1, X, y_f32, M, K, residual, &mrc)) return mrc;
     }
-    if (M > 8)
-        return gemm_int4_f16(st, Y, y_f32, X, W, (const uint16_t*)S, nullptr, nullptr, bias, M, N, K,
-                             residual);
+    if (M > 8) {
+        const xinfer_fused_desc one = {Y, W, S, bias, N};
+        return prefill_gemm(st, &one, 1, nullptr, nullptr, X, y_f32, M, K, residual);
+    }
     if (M == 1) {  // large N: the row-pair kernel (its 4-wave form for long K)
         const xinfer_fused_desc one = {Y, W, S, bias, N};
         int prc = XINFER_OK;
@@ -998,15 +998,7 @@ int fused_f16_impl(void* stream, const void* X0, const xinfer_fused_desc* descs,
         if (!pairm_linear(st, live, nd, X, false, M, K, false, &mrc)) return mrc;
         if (!mb_linear(st, live, nd, X, false, M, K, false, &mrc)) return mrc;
     }
-    if (M > 8) {  // one GEMM per descriptor
-        for (int i = 0; i < nd; ++i) {
-            const xinfer_fused_desc& q = live[i];
-            const int rc = gemm_int4_f16(st, q.Y, false, X, q.W_int4, (const uint16_t*)q.scales, nullptr,
-                                         nullptr, q.bias, M, q.N, K);
-            if (rc) return rc;
-        }
-        return XINFER_OK;
-    }
+    if (M > 8) return prefill_gemm(st, live, nd, nullptr, nullptr, X, false, M, K, false);
     if (M == 1) {  // large N: the row-pair kernel (the norm, if any, in its X staging)
         int prc = XINFER_OK;
         if (!pair_linear(st, live, nd, X, false, K, false, norm_in_kernel ? norm_w : nullptr, eps, &prc))
@@ -1049,9 +1041,10 @@ int swiglu_f16_impl(void* stream, void* Y, const void* X0, const uint8_t* W_gate
         if (!mb_swiglu(st, Y, X, W_gate, scales_gate, W_up, scales_up, M, N, K, &mrc))
             return mrc;
     }
-    if (M > 8)
-        return gemm_int4_f16(st, Y, false, X, W_gate, (const uint16_t*)scales_gate, W_up,
-                             (const uint16_t*)scales_up, nullptr, M, N, K);
+    if (M > 8) {
+        const xinfer_fused_desc one = {Y, W_gate, scales_gate, nullptr, N};
+        return prefill_gemm(st, &one, 1, W_up, (const uint16_t*)scales_up, X, false, M, K, false);
+    }
     if (M == 1 && swiglu_pair_on()) {  // large N: the row-pair kernel (the norm, if any, in its X staging)
         int prc = XINFER_OK;
         if (!pair_swiglu(st, Y, X, W_gate, scales_gate, W_up, scales_up, N, K, norm_in_kernel ? norm_w : nullptr,

@@ -11,7 +11,9 @@
 //
 // The array holds kSplitSlots independent slots (partials + arrival
 // counters), 32 x (4 MiB + 16 KiB) = 128.5 MiB on every device the library
-// runs on.  A slot belongs to one stream of a device until
+// runs on; the first 8 slots also have 64 MiB each for the prefill GEMM's
+// partial tiles (512 MiB: room for two partial tiles of 128 x 256 per CU).
+// A slot belongs to one stream of a device until
 // xinfer_stream_release gives it back: calls on one stream run in order, so
 // they never share a slot concurrently, and calls on different streams use
 // different slots.  Every counter is zero at load time and is returned to
@@ -29,6 +31,9 @@ constexpr size_t kSplitPartialFloats = (size_t)1 << 20;  // 4 MiB of FP32 partia
 constexpr int kSplitCounters = 4096;                       // tile ranges per slot
 
 __device__ __align__(256) float g_splitk_partials[kSplitSlots][kSplitPartialFloats];
+constexpr int kSkSlots = 8;                               // streams with room for the prefill GEMM's
+constexpr size_t kSkPartialFloats = (size_t)1 << 24;      // partial tiles: 64 MiB each
+__device__ __align__(256) float g_sk_partials[kSkSlots][kSkPartialFloats];
 __device__ __align__(256) uint32_t g_splitk_counters[kSplitSlots][kSplitCounters];
 }  // namespace xhip
 
@@ -40,6 +45,7 @@ struct DevSlots {
     bool resolved = false;
     float* partials = nullptr;    // device address of g_splitk_partials on this device
     uint32_t* counters = nullptr; // device address of g_splitk_counters on this device
+    float* sk = nullptr;          // device address of g_sk_partials on this device
     int nused = 0;
     hipStream_t owner[xhip::kSplitSlots] = {};
     bool released[xhip::kSplitSlots] = {};
@@ -48,25 +54,29 @@ std::mutex g_mu;
 DevSlots g_devs[kMaxDev];
 }  // namespace
 
-// The split-K slot of `st` on the current device: its partials (capacity in
-// floats) and counters (count).  Returns false when the device's slots are
-// all owned by other streams or the symbol lookup failed.
-bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint32_t** counters,
-                 int* ncounters) {
+namespace {
+
+// The slot of `st` on the current device, whose addresses go to *out; -1 when
+// the device's slots are all owned by other streams or the symbol lookup
+// failed.
+int slot_of(hipStream_t st, DevSlots* out) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return false;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return -1;
     std::lock_guard<std::mutex> lock(g_mu);
     DevSlots& d = g_devs[dev];
     if (!d.resolved) {
         void* pa = nullptr;
         void* ca = nullptr;
+        void* ga = nullptr;
         if (hipGetSymbolAddress(&pa, HIP_SYMBOL(xhip::g_splitk_partials)) != hipSuccess ||
-            hipGetSymbolAddress(&ca, HIP_SYMBOL(xhip::g_splitk_counters)) != hipSuccess || !pa || !ca) {
+            hipGetSymbolAddress(&ca, HIP_SYMBOL(xhip::g_splitk_counters)) != hipSuccess ||
+            hipGetSymbolAddress(&ga, HIP_SYMBOL(xhip::g_sk_partials)) != hipSuccess || !pa || !ca || !ga) {
             (void)hipGetLastError();
-            return false;
+            return -1;
         }
         d.partials = reinterpret_cast<float*>(pa);
         d.counters = reinterpret_cast<uint32_t*>(ca);
+        d.sk = reinterpret_cast<float*>(ga);
         d.resolved = true;
     }
     int slot = -1, freed = -1;
@@ -78,12 +88,27 @@ bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint3
         if (freed >= 0) {
             slot = freed;
         } else {
-            if (d.nused == xhip::kSplitSlots) return false;
+            if (d.nused == xhip::kSplitSlots) return -1;
             slot = d.nused++;
         }
         d.owner[slot] = st;
         d.released[slot] = false;
     }
+    out->partials = d.partials;
+    out->counters = d.counters;
+    out->sk = d.sk;
+    return slot;
+}
+
+}  // namespace
+
+// The split-K slot of `st` on the current device: its partials (capacity in
+// floats) and counters (count).  Returns false when there is none.
+bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint32_t** counters,
+                 int* ncounters) {
+    DevSlots d;
+    const int slot = slot_of(st, &d);
+    if (slot < 0) return false;
     *partials = d.partials + (size_t)slot * xhip::kSplitPartialFloats;
     *partial_floats = xhip::kSplitPartialFloats;
     *counters = d.counters + (size_t)slot * xhip::kSplitCounters;
@@ -91,6 +116,19 @@ bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint3
     return true;
 }
 
+// The same slot for the prefill GEMM (gemm_sk_int4.hip): the first
+// kSkSlots slots have 64 MiB for its partial tiles, the others make do with
+// the slot's 4 MiB.
+bool sk_slot(hipStream_t st, float** partials, size_t* partial_floats) {
+    DevSlots d;
+    const int slot = slot_of(st, &d);
+    if (slot < 0) return false;
+    const bool big = slot < xhip::kSkSlots;
+    *partials = big ? d.sk + (size_t)slot * xhip::kSkPartialFloats
+                    : d.partials + (size_t)slot * xhip::kSplitPartialFloats;
+    *partial_floats = big ? xhip::kSkPartialFloats : xhip::kSplitPartialFloats;
+    return true;
+}
 
 // Gives the split-K slot of `st` on the current device back (its counters
 // are zero once the stream's work has finished).
