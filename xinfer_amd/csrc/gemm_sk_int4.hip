@@ -261,8 +261,13 @@ __global__ __launch_bounds__(64 * sk::kWaves) void gemm_sk_int4_kernel(const SkP
         const uint16_t* sp = nullptr;
         uint32_t off[CPW];
         int to = 0;  // its place in the ring
-        auto wchunk = [](int row, int ch) {  // where a row's chunk is stored
-            return KW == 2 ? ch ^ (row & 7) : ch ^ ((row >> 1) & 3);
+        // Where a row's chunk is stored: LDS serves 16 lanes of 16 bytes a cycle from
+        // 64 banks, so a chunk of 16 consecutive rows takes every place of 256 bytes
+        // once (with the order of 8 rows repeated, half of the LDS cycles were bank
+        // conflicts).
+        auto xchunk = [](int row, int ch) { return ch ^ (row & 7) ^ ((row >> 3) & 1); };
+        auto wchunk = [&](int row, int ch) {
+            return KW == 2 ? xchunk(row, ch) : ch ^ ((row >> 2) & 3);
         };
         // Lane-dependent addresses of rare work are computed where they are used
         // and not kept in registers through the loop.
@@ -290,7 +295,7 @@ __global__ __launch_bounds__(64 * sk::kWaves) void gemm_sk_int4_kernel(const SkP
                     const int gq = q / (8 * MT), qq = q - gq * (8 * MT);   // group of the step, copy of the group
                     const int rg = qq / (4 * MT), rb = qq - rg * (4 * MT);
                     const int xr = min(m0 + rb * 8 + (lane >> 3), M - 1);
-                    off[j] = ((uint32_t)xr * (uint32_t)p.K + 128u * gq + 64u * rg + 8u * ((lane & 7) ^ (lane >> 3))) * 2u;
+                    off[j] = ((uint32_t)xr * (uint32_t)p.K + 128u * gq + 64u * rg + 8u * xchunk(rb * 8 + (lane >> 3), lane & 7)) * 2u;
                 }
                 const int v = (role * 64 + lane) % bn(MT);
                 sp = ((SWIGLU && (v & 16)) ? d.S2 : d.S) + (size_t)row_of(v) * ng;
@@ -332,7 +337,7 @@ __global__ __launch_bounds__(64 * sk::kWaves) void gemm_sk_int4_kernel(const SkP
         int xa[4], wa[2];
 #pragma unroll
         for (int d = 0; d < 4; ++d)
-            xa[d] = kw * (MT * 8192) + (li >> 3) * 1024 + (li & 7) * 128 + (((4 * lh + d) ^ (li & 7)) * 16);
+            xa[d] = kw * (MT * 8192) + (li >> 3) * 1024 + (li & 7) * 128 + xchunk(li, 4 * lh + d) * 16;
 #pragma unroll
         for (int j = 0; j < 2; ++j)
             wa[j] = off_w(MT) + (cgr * 32 + li) * (64 * KW) + 16 * wchunk(li, 4 * kw + 2 * j + lh);
@@ -341,51 +346,62 @@ __global__ __launch_bounds__(64 * sk::kWaves) void gemm_sk_int4_kernel(const SkP
         // One step: k = 64 j + 32 lh + 8 d of dword d of weight chunk j.  16-k
         // steps of two row tiles at a time, the operands of the next one read and
         // decoded between the MFMAs; the second pair of row tiles reuses the
-        // decoded weights.  The copies of the step after next go out one at a
-        // time between them: a wave waits at a copy until the address unit takes
-        // it, so all of them at the start of the step would hold every wave for as
-        // long as the unit needs for the block's copies (measured: a step took the
-        // sum of its copies' and its arithmetic's time).
-        auto compute = [&](int xat, int wat, float s) {
-            constexpr int P0 = MT < 2 ? MT : 2, P1 = MT - P0;
+        // decoded weights.  The first operands of the next step are read at this
+        // one's end, so no wave starts a step with a wait for LDS.
+        // The copies of a later step go out one or two at a time between the
+        // first MFMAs: a wave waits at a copy until the address unit takes it,
+        // so all of them at the start of the step would hold every wave for as
+        // long as the unit needs for the block's copies (measured: a step then
+        // took the sum of its copies' and its arithmetic's time).
+        constexpr int P0 = MT < 2 ? MT : 2, P1 = MT - P0;
+        u32x4 w[2];
+        f16x8 b[P1 > 0 ? 8 : 2];
+        f16x8 a[2][2];
+        auto opread = [&](const unsigned char* xs, int k, int mt0, int n, int into) {
+#pragma unroll
+            for (int t = 0; t < n; ++t)
+                a[into][t] = *reinterpret_cast<const f16x8*>(xs + xa[k & 3] + ((k >> 2) * MT + mt0 + t) * 4096);
+        };
+        auto first = [&](int xat, int wat) {
+            w[0] = *reinterpret_cast<const u32x4*>(smem + wat + wa[0]);
+            opread(smem + xat, 0, 0, P0, 0);
+            w[1] = *reinterpret_cast<const u32x4*>(smem + wat + wa[1]);
+        };
+        auto mfma = [&](f16x8 x, f16x8 y, f32x16 c, bool zero) {
+            if (zero) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) c[e] = 0.0f;
+            }
+            return __builtin_amdgcn_mfma_f32_32x32x16_f16(x, y, c, 0, 0, 0);
+        };
+        // `mid` runs once all copies of the step are out
+        auto compute = [&](int xat, float s, auto mid, auto next) {
             const unsigned char* xs = smem + xat;
-            const unsigned char* ws = smem + wat;
-            u32x4 w[2];
-            f16x8 b[P1 > 0 ? 8 : 2];
-            f16x8 a[2][2];
             f32x16 pa[P0], pb[P1 > 0 ? P1 : 1];
-            auto opread = [&](int k, int mt0, int n, int to) {
-#pragma unroll
-                for (int t = 0; t < n; ++t)
-                    a[to][t] = *reinterpret_cast<const f16x8*>(xs + xa[k & 3] + ((k >> 2) * MT + mt0 + t) * 4096);
-            };
-            auto mfma = [&](f16x8 x, f16x8 y, f32x16 c, bool zero) {
-                if (zero) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) c[e] = 0.0f;
-                }
-                return __builtin_amdgcn_mfma_f32_32x32x16_f16(x, y, c, 0, 0, 0);
-            };
-            w[0] = *reinterpret_cast<const u32x4*>(ws + wa[0]);
-            opread(0, 0, P0, 0);
-            w[1] = *reinterpret_cast<const u32x4*>(ws + wa[1]);
+            constexpr int CPK = P1 > 0 ? 1 : 2;  // copies per 16-k step
+            static_assert(CPW <= (P1 > 0 ? 8 : 8), "copies before the middle");
             b[0] = sk_decode8(w[0][0]);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
                 const int cur = k & 1;
-                if (k < 7) opread(k + 1, 0, P0, cur ^ 1);
-                else if (P1) opread(0, P0, P1, cur ^ 1);
+                if (k < 7) opread(xs, k + 1, 0, P0, cur ^ 1);
+                else if (P1) opread(xs, 0, P0, P1, cur ^ 1);
+                else next();
 #pragma unroll
                 for (int t = 0; t < P0; ++t) pa[t] = mfma(a[cur][t], b[P1 > 0 ? k : cur], pa[t], k == 0);
-                if (k < CPW) copy(k);
+#pragma unroll
+                for (int c = 0; c < CPK; ++c)
+                    if (k * CPK + c < CPW) copy(k * CPK + c);
                 if (k < 7) b[P1 > 0 ? k + 1 : cur ^ 1] = sk_decode8(w[(k + 1) >> 2][(k + 1) & 3]);
                 __builtin_amdgcn_sched_barrier(0);
+                if (k == (P1 > 0 ? 7 : 3)) mid();
             }
             if constexpr (P1 > 0) {
 #pragma unroll
                 for (int k = 0; k < 8; ++k) {
                     const int cur = k & 1;
-                    if (k < 7) opread(k + 1, P0, P1, cur ^ 1);
+                    if (k < 7) opread(xs, k + 1, P0, P1, cur ^ 1);
+                    else next();
 #pragma unroll
                     for (int t = 0; t < P1; ++t) pb[t] = mfma(a[cur][t], b[k], pb[t], k == 0);
 #pragma unroll
@@ -469,62 +485,71 @@ __global__ __launch_bounds__(64 * sk::kWaves) void gemm_sk_int4_kernel(const SkP
             advance();
             __builtin_amdgcn_sched_barrier(0);
         };
+        uint16_t s_next;  // X waves: the scale of the step after the one in use
         if constexpr (xwave) {
             const uint16_t sa = scale_load();
             ahead();
-            const uint16_t sb = scale_load();
+            s_next = scale_load();
             ahead();
             sbuf[role * 64 + lane] = sa;
-            sbuf[kScales + role * 64 + lane] = sb;
         } else {
             for (int k = 0; k < RW - 1; ++k) ahead();
         }
-        auto landed = [&]() {  // this wave's copies of the next step, and of the scales after it
+        auto landed = [&]() {  // this wave's copies of the next step
             if constexpr (xwave) {
                 XHIP_SK_VMCNT(XPW);
             } else {
                 XHIP_SK_VMCNT((RW - 2) * WPW);
             }
         };
+        auto barrier = [&]() {
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        };
         landed();
-        __builtin_amdgcn_s_waitcnt(0xC07F);  // the scales are stored
+        __builtin_amdgcn_s_waitcnt(0xC07F);  // the scale is stored
+        barrier();
+        first(0, 0);
         for (;;) {
-            asm volatile("" ::: "memory");
-            __builtin_amdgcn_s_barrier();  // ... of every wave; the step before this one is free
-            asm volatile("" ::: "memory");
+            // here every wave is past the step before this one, whose places the
+            // copies may take
+            const int xnx = xat == 2 * XB ? 0 : xat + XB;
+            const int wnx = wat == (RW - 1) * WB ? 0 : wat + WB;
+            const int snx = sat == 2 * kScales ? 0 : sat + kScales;
             __builtin_amdgcn_sched_barrier(0);
-            uint16_t s2;
-            if constexpr (xwave) s2 = scale_load();
-            __builtin_amdgcn_sched_barrier(0);  // older than the step's copies
+            // The middle of a step: the next one's copies and scales are in LDS.
+            auto mid = [&]() {
+                landed();
+                if constexpr (xwave) sbuf[snx + role * 64 + lane] = s_next;
+                __builtin_amdgcn_s_waitcnt(0xC07F);
+                barrier();
+                if constexpr (xwave) s_next = scale_load();
+                advance();
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            auto next = [&]() { first(xnx, wnx); };
             if (KW == 1 || g < ng) {
-                compute(xat, wat, h2f(sbuf[sat + kw * bn(MT) + cgr * 32 + li]));
+                compute(xat, h2f(sbuf[sat + kw * bn(MT) + cgr * 32 + li]), mid, next);
             } else {  // a dead group is not read
 #pragma unroll
                 for (int j = 0; j < CPW; ++j) copy(j);
+                mid();
+                next();
             }
             __builtin_amdgcn_sched_barrier(0);
-            landed();
-            const int sto = sat == 0 ? 2 * kScales : sat - kScales;
-            if constexpr (xwave) sbuf[sto + role * 64 + lane] = s2;
-            advance();
-            __builtin_amdgcn_s_waitcnt(0xC07F);  // this step's operand reads, the scale's store
             g += KW;
             if (--i == 0) {
                 unsigned char* const used = smem + xat;  // free once every wave is past its reads
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
+                barrier();
                 if (KW > 1) {
                     sum_waves(used);
                     __builtin_amdgcn_s_waitcnt(0xC07F);  // the sums are read before staged rows take their place
-                    asm volatile("" ::: "memory");
-                    __builtin_amdgcn_s_barrier();
-                    asm volatile("" ::: "memory");
+                    barrier();
                 }
-                if (end == ns) {
-                    if (kw == 0) store_tile(ct, used);
-                } else {
-                    if (kw == 0) store_piece(ct * ns + cg == u0 ? 0 : 1);
+                if (kw == 0) {
+                    if (end == ns) store_tile(ct, used);
+                    else store_piece(ct * ns + cg == u0 ? 0 : 1);
                 }
                 rem -= end;
                 if (rem <= 0) break;
@@ -535,9 +560,10 @@ __global__ __launch_bounds__(64 * sk::kWaves) void gemm_sk_int4_kernel(const SkP
                 clear();
                 __builtin_amdgcn_s_waitcnt(0xC07F);  // reads of the staged rows
             }
-            xat = xat == 2 * XB ? 0 : xat + XB;
-            wat = wat == (RW - 1) * WB ? 0 : wat + WB;
-            sat = sat == 2 * kScales ? 0 : sat + kScales;
+            barrier();
+            xat = xnx;
+            wat = wnx;
+            sat = snx;
         }
         XHIP_SK_VMCNT(0);  // no copy is left in flight
     };
