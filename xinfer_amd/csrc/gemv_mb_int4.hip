@@ -808,9 +808,18 @@ struct MbPlan {
 
 // Plan a small-batch launch.  Returns false when the shape does not fit the
 // kernel (X slice of one group per block beyond LDS) or M is outside 2..8.
-//   ks:  the smallest number of k-slices whose X slice fits the LDS budget,
-//        raised while the tile ranges alone cannot give every CU `bpc`
-//        blocks (short N, long K); argmax keeps ks = 1.
+//   ks:  the smallest number of k-slices whose X slice fits the LDS budget;
+//        where that is more than one, raised while the tile ranges alone
+//        cannot give every CU `bpc` blocks (short N, long K), at M <= 8.  A
+//        shape that one slice holds keeps it: the combine across blocks takes
+//        about 4 us (partials to memory, a release per block, the last one's
+//        reads), and fewer, longer blocks cost less.  Measured with the raise
+//        -> without, K x N: 1024 x 3000 M = 3 / 8 / 16 10.0 / 10.1 / 11.1 ->
+//        6.1 / 6.3 / 6.6 us, 640 x 1500 M = 8 9.6 -> 6.3, 3456 x 3500 M = 8
+//        11.3 -> 7.4, 5120 x 1024 M = 8 12.1 -> 8.9; with more than one slice
+//        anyway, 6144 x 5120 M = 5 / 8 13.0 / 13.3 -> 14.5 / 15.6, 9728 x
+//        2560 M = 8 12.7 -> 15.5 (raise kept), at M = 12 13.6 -> 13.3 and
+//        17408 x 1024 M = 12 15.9 -> 13.9 (not kept).  argmax keeps ks = 1.
 //   tiles per block: the tiles spread evenly over cus * bpc / ks ranges.
 //   kw:  waves per run of tiles, splitting the slice's groups (every wave
 //        has a tile of its run): the smallest power of two that gives at
@@ -902,7 +911,8 @@ bool plan_mb(MbParams& p, MbPlan& pl, size_t ws_cap, int64_t cnt_cap, bool raise
         tiles_blk = (tiles_total + rt - 1) / rt;
         ranges = 0;
         for (int i = 0; i < p.ndesc; ++i) ranges += ((p.d[i].N + 15) / 16 + tiles_blk - 1) / tiles_blk;
-        if (pass == 0 && ov.ks <= 0 && ov.raise != 0 && raise_ok && EPI != MB_ARGMAX && ranges * ks < target) {
+        if (pass == 0 && ov.ks <= 0 && ov.raise != 0 && raise_ok && EPI != MB_ARGMAX && ks > 1 && mr < 16 &&
+            ranges * ks < target) {
             int ks2 = (int)(target / ranges);
             if (ks2 > ng) ks2 = ng;
             if (ks2 > ks) { ks = ks2; continue; }
