@@ -37,7 +37,8 @@ def _check16(y, ref):
 
 @pytest.mark.parametrize("M,N,K", [(17, 1, 128), (17, 130, 256), (32, 257, 384), (33, 128, 3456), (64, 600, 640),
                                    (65, 255, 1024), (96, 72, 2176), (97, 300, 128), (128, 1000, 896),
-                                   (129, 264, 1152), (160, 48, 5120), (257, 520, 384), (512, 136, 640)])
+                                   (129, 264, 1152), (160, 48, 5120), (257, 520, 384), (512, 136, 640),
+                                   (9, 9001, 9088), (16, 15632, 5248)])  # M <= 16: long K, many weights
 def test_plain_forms(M, N, K):
     import torch
     from xinfer_amd import ops
