@@ -119,7 +119,7 @@ __device__ __forceinline__ f16x8 sk_decode8(uint32_t w) {
 // e: column li, row 8 (e / 4) + 4 lh + e % 4) at row m0 and output column n0.
 // SwiGLU: columns 0-15 are gate, 16-31 up rows of 16 output columns.  `st`:
 // kOutWave bytes of LDS of this wave.
-template <bool SWIGLU, typename OutT>
+template <bool SWIGLU, typename OutT, bool HALVES>
 __device__ __forceinline__ void sk_store(const SkDesc& d, const f32x16& sum, int m0, int n0, int M, bool residual,
                                          unsigned char* st, int lane) {
     using namespace sk;
@@ -130,22 +130,38 @@ __device__ __forceinline__ void sk_store(const SkDesc& d, const f32x16& sum, int
     const int col = SWIGLU ? (lane & 15) : li;
     const float bn = (!SWIGLU && d.bias && n0 + col < N) ? d.bias[n0 + col] : 0.0f;
     OutT* const Y = reinterpret_cast<OutT*>(d.Y);
-    float v[16];
+    // SwiGLU: lanes 16 apart hold gate and up of the same outputs.  HALVES:
+    // each of the two takes half of them (in the second launch, whose waves
+    // do little else: N = 3000, K = 2176, M = 40 18.9 -> 17.9 us, N = 1100,
+    // K = 5120, M = 77 22.8 -> 20.2); in the main kernel, where it costs the
+    // loop its registers (N = 17408, K = 5120, M = 60 45.7 -> 52.8), the lane
+    // with the gate row computes all 16.
+    constexpr bool BOTH = SWIGLU && HALVES;
+    constexpr int NV = BOTH ? 8 : 16;
+    const int up16 = BOTH ? (lane & 16) : 0;  // the upper half's rows
+    const bool live = !SWIGLU || BOTH || !(lane & 16);
+    auto row_of = [&](int e) { return 8 * (e >> 2) + 4 * lh + (e & 3) + up16; };
+    float v[NV];
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        v[e] = sum[e] + bn;
-        if (SWIGLU) {
+    for (int e = 0; e < NV; ++e) {
+        if constexpr (BOTH) {
+            const float mine = up16 ? sum[e + 8] : sum[e];
+            const float other = __shfl_xor(up16 ? sum[e] : sum[e + 8], 16);
+            const float g = up16 ? other : mine, u = up16 ? mine : other;
+            v[e] = g / (1.0f + expf(-g)) * u;
+        } else if constexpr (SWIGLU) {
             const float u = __shfl_xor(sum[e], 16);
-            v[e] = v[e] / (1.0f + expf(-v[e])) * u;
+            v[e] = sum[e] / (1.0f + expf(-sum[e])) * u;
+        } else {
+            v[e] = sum[e] + bn;
         }
     }
-    const bool live = !SWIGLU || !(lane & 16);
     if constexpr (sizeof(OutT) == 2) {
         if (d.y16) {  // whole 16-byte pieces of rows, through LDS
             if (live) {
 #pragma unroll
-                for (int e = 0; e < 16; ++e)
-                    *reinterpret_cast<f16*>(st + out_at(8 * (e >> 2) + 4 * lh + (e & 3), col >> 3) + 2 * (col & 7)) = (f16)v[e];
+                for (int e = 0; e < NV; ++e)
+                    *reinterpret_cast<f16*>(st + out_at(row_of(e), col >> 3) + 2 * (col & 7)) = (f16)v[e];
             }
             constexpr int CH = COLS / 8;  // pieces of a row
             constexpr int RPS = 64 / CH;  // rows per store
@@ -174,8 +190,8 @@ __device__ __forceinline__ void sk_store(const SkDesc& d, const f32x16& sum, int
         }
     }
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-        const int m = m0 + 8 * (e >> 2) + 4 * lh + (e & 3);
+    for (int e = 0; e < NV; ++e) {
+        const int m = m0 + row_of(e);
         if (live && m < M && n0 + col < N) {
             OutT* y = Y + (size_t)m * N + n0 + col;
             if (sizeof(OutT) == 2 && residual)
@@ -459,7 +475,7 @@ __global__ __launch_bounds__(64 * sk::kWaves) void gemm_sk_int4_kernel(const SkP
             const int n0 = (ct - d.tile_begin) * (CG * COLS) + cgr * COLS;
 #pragma unroll
             for (int mt = 0; mt < MT; ++mt)
-                sk_store<SWIGLU, OutT>(d, acc[mt], mb * BM + mt * 32, n0, M, p.residual != 0, st + cgr * kOutWave, lane);
+                sk_store<SWIGLU, OutT, false>(d, acc[mt], mb * BM + mt * 32, n0, M, p.residual != 0, st + cgr * kOutWave, lane);
         };
 
         int ct = pt, cg = pg;
@@ -617,7 +633,7 @@ __global__ __launch_bounds__(256) void gemm_sk_sum_kernel(const SkParams p) {
     }
     const int ct = p.mb == 1 ? t : sk_div(t, p.mb, p.inv_mb);
     const SkDesc& d = sk_desc(p, ct);
-    sk_store<SWIGLU, OutT>(d, acc, (t - ct * p.mb) * (32 * MT) + mt * 32, (ct - d.tile_begin) * (CG * COLS) + cgr * COLS,
+    sk_store<SWIGLU, OutT, true>(d, acc, (t - ct * p.mb) * (32 * MT) + mt * 32, (ct - d.tile_begin) * (CG * COLS) + cgr * COLS,
                            p.M, p.residual != 0, smem + wave * kOutWave, lane);
 }
 
