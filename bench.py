@@ -573,7 +573,7 @@ def run_suite(torch, dev, ops, synth, args, log, want, graph):
         record("cfg4_prefill_exact_dequant_m512_n17408_k5120" if exact_route else "cfg4_prefill_m512_n17408_k5120",
                {"M": M, "N": N, "K": K, "us": round(e * 1e6, 2), "TFLOPs": round(fl / e / 1e12, 1),
                 "frac_fp16_mfma": round(fl / e / 1e12 / FP16_PEAK_TFLOPS, 4),
-                "kernel": ("xhip::gemm_int4_mfma_kernel<EXACT> (exact q, FP32 group scale; 128-row blocks)"
+                "kernel": ("xhip::gemm_sk_int4_kernel (exact q, FP32 group scale; steps cut evenly over the CUs)"
                            if exact_route else
                            "xhip::gemm_ws_int4_kernel (256x136 blocks; 4 MFMA waves copying their own X "
                            "rows, 4 weight-decode waves; B = fp16(q*s))")})

@@ -19,13 +19,14 @@
 // 41.2 us.)
 //
 // What bounds it: at M <= 64 the weights' arrival and the decode (12 VALU per
-// packed dword, two waves per SIMD), at larger M the LDS operand reads (each
-// feeds one 32-column MFMA) together with the MFMAs.  N = 17408, K = 5120,
-// M = 17 / 64 / 128: 21.7 / 27.3 / 41.1 us = 2.1 / 1.6 / 1.1 TB/s of weights,
-// 110 / 418 / 555 TFLOP/s (the 128-row GEMM with a block per tile and rounded
-// weights that it replaced: 49.3 / 55.0 / 68.2); N = 5120, K = 17408, M = 23 /
-// 512: 23.2 / 106 us (157 / 201); K = 3456, N = 5003, M = 200, fp32 outputs:
-// 26.6 us (214 as GEMV slabs of 8 rows).  Before the run cut, those long-K,
+// packed dword, two waves per SIMD), at larger M the MFMAs at the clock that
+// they leave (1.46 GHz at M = 128, N = 69632, matrix cores busy 53 %).
+// N = 17408, K = 5120, M = 17 / 64 / 128: 21.9 / 26.7 / 40.8 us = 2.0 / 1.7 /
+// 1.1 TB/s of weights, 138 / 427 / 559 TFLOP/s (the 128-row GEMM with a block
+// per tile and rounded weights that it replaced: 49.3 / 55.0 / 68.2);
+// N = 5120, K = 17408, M = 23 / 512: 23.2 / 104 us (157 / 201); K = 3456,
+// N = 5003, M = 200, fp32 outputs: 27.0 us (214 as GEMV slabs of 8 rows).
+// Before the run cut, those long-K,
 // small-N shapes left two thirds of the CUs without a block.
 
 #include <stdlib.h>

@@ -14,7 +14,7 @@
 // B = fp16(q * s): q (an integer in [-8, 7]) is exact in fp16 and the
 // product is rounded once (relative error <= 2^-11), well inside the fp16
 // output's own rounding and the BASELINE bound; fp32 outputs take the exact
-// kernel in gemm_int4.hip.
+// kernel in gemm_sk_int4.hip.
 
 #include <stdlib.h>
 
