@@ -24,15 +24,19 @@
  * 359, 513) M, N or K <= 0 is a no-op that returns XINFER_OK.
  *
  * No projection entry point allocates device memory or synchronises: the
- * first call of any shape can be captured into a hipGraph.  The small-batch
- * kernel's cross-block split-K partials live in a static device array that
- * the code object loader places with the library's kernels: 32 slots of
- * 4 MiB + 16 KiB (128.5 MiB) on every device the library runs on, one
- * owned by each stream that calls until xinfer_stream_release gives it
- * back; the first 8 also hold 64 MiB each (512 MiB) for the partial sums of
- * the prefill GEMM (M > 16); with every slot owned a call plans without the cross-block split
- * (correct, slower).  Calls on different streams may therefore overlap.  A
- * graph holds the slot of the stream it was captured on: replays of graphs
+ * first call of any shape can be captured into a hipGraph.  Partial sums
+ * that cross blocks live in static device arrays that the code object loader
+ * places: for the small-batch kernel's split of K 32 slots of 4 MiB + 16 KiB
+ * (128.5 MiB), with the library's kernels; for the prefill GEMM 64 MiB for
+ * each of up to 32 streams whose calls leave partial tiles, in groups of
+ * 1, 1, 2, 4, 8 and 16 placed when the first of them is needed (25 ms per
+ * area then; a program that only decodes holds none).  A stream owns its slot
+ * and its area, on every device it calls on, until xinfer_stream_release
+ * gives them back; with every one owned a call plans without the cross-block
+ * split (correct, slower, other rounding of the FP32 sums).  Calls on
+ * different streams may therefore overlap.  A
+ * graph holds the slot and the area of the stream it was captured on: replays
+ * of graphs with decode or prefill calls
  * captured on one stream must not overlap each other or that stream's work
  * (a decode-step graph replayed in order on its own stream, as the
  * reference's DecodeGraph does, src/targets/qwen3_8/decode_graph.cpp:9-12,
@@ -69,9 +73,10 @@ const char* xinfer_status_string(int status);
 /* No counterpart in the reference (its queues are created once per
  * DeviceContext and never destroyed).  For long-running callers that create
  * and destroy streams: waits for `stream`'s work, then gives back its
- * split-K slot and frees its argmax scratch on the current device, so a
- * later stream can take them.  Call it before hipStreamDestroy; without it a
- * destroyed stream keeps its slot until the process ends. */
+ * split-K slot and its area for partial tiles and frees its argmax scratch on
+ * the current device, so a later stream can take them.  Call it before
+ * hipStreamDestroy; without it a destroyed stream keeps its slot and area until
+ * the process ends. */
 int xinfer_stream_release(void* stream);
 
 /* Library version string, e.g. "xinfer_hip 0.1.0 gfx950". */

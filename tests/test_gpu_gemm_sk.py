@@ -79,34 +79,45 @@ def test_swiglu(M, N, K):
     _check16(y, oracle.swiglu_int4(oracle.f16_to_f32(Xb), W, S, U, T, M, N, K, nthreads=cpu_threads()))
 
 
-def test_streams_past_the_scratch_slots():
-    """Calls on more streams than have scratch for partial sums: whole-tile
-    runs there, and on every stream the same values within the bound, also
-    with the calls of several streams in flight."""
+def test_streams_past_the_areas():
+    """Cut calls in flight on more streams than have areas for partial tiles,
+    each on X of its own: every result within the bound of its own oracle
+    values, and on the first streams, which have an area, also the bits that
+    the same call gives on the current stream."""
+    import ctypes
     import torch
     from xinfer_amd import _lib, ops
-    M, N, K = 40, 384, 2560
-    W, S, Xb = _inputs(M, N, K, 5)
-    dW, dS, dX = to_dev(W), f16_dev(S), f16_dev(Xb)
-    ref = oracle.linear_int4(oracle.f16_to_f32(Xb), W, S, M, N, K, nthreads=cpu_threads())
-    torch.cuda.synchronize()
+    M, N, K = 512, 136, 640  # 20 runs over 4 tiles; 4 runs of whole tiles without an area
+    W, S, _ = _inputs(M, N, K, 5)
+    Xs = [synth.activations(100 + i, M, K) for i in range(36)]
+    dW, dS, dXs = to_dev(W), f16_dev(S), [f16_dev(x) for x in Xs]
+    refs = [oracle.linear_int4(oracle.f16_to_f32(x), W, S, M, N, K, nthreads=cpu_threads()) for x in Xs]
+    solo = torch.full((36, M, N), float("nan"), device="cuda")
+    for y, x in zip(solo, dXs):
+        ops.linear_int4(y, x, dW, dS, None, M, N, K)
     # raw streams: torch hands out its 32 pooled ones over and over
-    import ctypes
     hip = ctypes.CDLL("libamdhip64.so")
     raw = []
     for _ in range(36):
         h = ctypes.c_void_p()
         assert hip.hipStreamCreate(ctypes.byref(h)) == 0
         raw.append(h)
-    ys = [torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda") for _ in raw]
+    ys = torch.full((3, 36, M, N), float("nan"), device="cuda")
     torch.cuda.synchronize()
-    for h, y in zip(raw, ys):
-        ops.linear_int4(y, dX, dW, dS, None, M, N, K, stream=h.value)
+    for r in range(3):  # a stream's calls differ from one to the next
+        for i, h in enumerate(raw):
+            j = (i + r) % 36
+            ops.linear_int4(ys[r, i], dXs[j], dW, dS, None, M, N, K, stream=h.value)
     torch.cuda.synchronize()
-    for h, y in zip(raw, ys):
-        _check16(y, ref)
+    for h in raw:
         assert _lib.load_library().xinfer_stream_release(h) == 0
         assert hip.hipStreamDestroy(h) == 0
+    for r in range(3):
+        for i in range(36):
+            j = (i + r) % 36
+            assert np.abs(to_np(ys[r, i]) - refs[j]).max() <= 1e-4, (r, i)
+            if i < 24:  # 32 areas, a few of them other tests' streams'
+                assert torch.equal(ys[r, i], solo[j]), (r, i)
 
 
 def test_graph_replay():

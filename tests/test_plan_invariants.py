@@ -56,3 +56,17 @@ def test_prefill_gemm_split(tmp_path):
     run = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     print(run.stdout)
     assert run.returncode == 0, run.stdout[-2000:]
+
+
+@pytest.mark.skipif(_hipcc() is None, reason="hipcc not available")
+def test_scratch_owners(tmp_path):
+    """Who owns the split-K slots and the prefill GEMM's areas."""
+    exe = str(tmp_path / "scratch_check")
+    build = subprocess.run([_hipcc(), "-O1", "-std=c++17", "--offload-arch=gfx950",
+                            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                            os.path.join(HERE, "scratch_check.hip"), "-o", exe],
+                           capture_output=True, text=True, timeout=900)
+    assert build.returncode == 0, build.stderr[-2000:]
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    print(run.stdout)
+    assert run.returncode == 0, run.stdout[-2000:]

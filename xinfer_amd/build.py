@@ -24,6 +24,8 @@ ARCH = "gfx950"
 
 SOURCES = ["gemv_int4.hip", "gemv_pair_int4.hip", "gemv_mb_int4.hip", "argmax.hip", "misc.hip", "crc64.hip",
            "artifact.hip", "scratch.hip", "noalloc.hip", "gemm_ws_int4.hip", "gemm_sk_int4.hip"]
+# compiled once per group of areas, each a code object that is placed by itself
+AREAS_SRC, AREA_GROUPS = "sk_areas.hip", 6
 
 # -packed-fp32-ops: keep the compiler from forming v_pk_{add,mul,fma}_f32
 # (packed fp16 ops are unaffected).
@@ -38,9 +40,13 @@ def hipcc() -> str:
     return os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "bin", "hipcc")
 
 
-def _compile(src: str) -> str:
-    obj = os.path.join(BUILD_DIR, os.path.splitext(src)[0] + ".o")
-    cmd = [hipcc(), *HIPCC_FLAGS, "-c", os.path.join(CSRC, src), "-o", obj]
+def _compile(src: str, group: int | None = None) -> str:
+    stem = os.path.splitext(src)[0]
+    obj = os.path.join(BUILD_DIR, stem + (".o" if group is None else f"_{group}.o"))
+    # the host's stand-ins for the areas (2 GiB of .bss, never touched) lie past
+    # the reach of 32-bit relocations
+    extra = [] if group is None else [f"-DXHIP_SK_GROUP={group}", "-Xarch_host", "-mcmodel=medium"]
+    cmd = [hipcc(), *HIPCC_FLAGS, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"hipcc failed for {src}:\n{r.stderr}")
@@ -51,7 +57,8 @@ def build(asm: bool = False) -> str:
     os.makedirs(BUILD_DIR, exist_ok=True)
     os.makedirs(OUT_DIR, exist_ok=True)
     with ThreadPoolExecutor(max_workers=min(8, len(SOURCES))) as ex:
-        objs = list(ex.map(_compile, SOURCES))
+        objs = list(ex.map(_compile, SOURCES + [AREAS_SRC] * AREA_GROUPS,
+                           [None] * len(SOURCES) + list(range(AREA_GROUPS))))
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc(), "-shared", "-fPIC", f"--offload-arch={ARCH}", *objs, "-o", tmp]
     r = subprocess.run(cmd, capture_output=True, text=True)

@@ -35,7 +35,7 @@
 #include <mutex>
 #include <type_traits>
 
-#include "common.h"
+#include "sk_areas.h"
 
 namespace xhip {
 
@@ -645,7 +645,7 @@ __global__ __launch_bounds__(256) void gemm_sk_sum_kernel(const SkParams p) {
 using namespace xhip;
 
 namespace xhip_host {
-bool sk_slot(hipStream_t st, float** partials, size_t* partial_floats);  // scratch.hip
+float* sk_area(hipStream_t st);  // scratch.hip
 int gemm_ws_linear(hipStream_t st, void* Y, const void* X, const uint8_t* W, const uint16_t* S, const float* bias,
                    int64_t M, int64_t N, int64_t K, bool residual, int* rc);  // gemm_ws_int4.hip
 }
@@ -736,10 +736,9 @@ int sk_launch(hipStream_t st, const xinfer_fused_desc* descs, int nd, const uint
               const void* X, bool y_f32, int64_t M, int64_t K, bool residual) {
     using namespace xhip_host;
     const bool swiglu = W2 != nullptr;
+    SkPlan pl = sk_plan(descs, nd, swiglu, M, K, kSkAreaFloats, num_cus());
     float* part = nullptr;
-    size_t part_floats = 0;
-    if (!sk_slot(st, &part, &part_floats)) part_floats = 0;
-    const SkPlan pl = sk_plan(descs, nd, swiglu, M, K, part_floats, num_cus());
+    if (!pl.whole && !(part = sk_area(st))) pl = sk_plan(descs, nd, swiglu, M, K, 0, num_cus());
     SkParams p = {};
     p.X = reinterpret_cast<const f16*>(X);
     p.part = part;

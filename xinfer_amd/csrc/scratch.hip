@@ -11,19 +11,22 @@
 //
 // The array holds kSplitSlots independent slots (partials + arrival
 // counters), 32 x (4 MiB + 16 KiB) = 128.5 MiB on every device the library
-// runs on; the first 8 slots also have 64 MiB each for the prefill GEMM's
-// partial tiles (512 MiB: room for two partial tiles of 128 x 256 per CU).
-// A slot belongs to one stream of a device until
+// runs on.  A slot belongs to one stream of a device until
 // xinfer_stream_release gives it back: calls on one stream run in order, so
 // they never share a slot concurrently, and calls on different streams use
 // different slots.  Every counter is zero at load time and is returned to
 // zero by the block that finishes its tile range, so a slot needs no
 // clearing between calls.  When every slot of a device is taken (more live
 // streams than slots) the caller plans without a cross-block split instead.
+//
+// The prefill GEMM's partial tiles have areas of their own (sk_areas.hip), 64
+// MiB for each stream whose calls leave such tiles, for up to kSkAreas streams
+// of a device, owned and given back as the slots are; with every area owned
+// its calls run as whole tiles.
 
 #include <mutex>
 
-#include "common.h"
+#include "sk_areas.h"
 
 namespace xhip {
 constexpr int kSplitSlots = 32;  // torch's stream pool alone hands out 32 streams per device
@@ -31,9 +34,6 @@ constexpr size_t kSplitPartialFloats = (size_t)1 << 20;  // 4 MiB of FP32 partia
 constexpr int kSplitCounters = 4096;                       // tile ranges per slot
 
 __device__ __align__(256) float g_splitk_partials[kSplitSlots][kSplitPartialFloats];
-constexpr int kSkSlots = 8;                               // streams with room for the prefill GEMM's
-constexpr size_t kSkPartialFloats = (size_t)1 << 24;      // partial tiles: 64 MiB each
-__device__ __align__(256) float g_sk_partials[kSkSlots][kSkPartialFloats];
 __device__ __align__(256) uint32_t g_splitk_counters[kSplitSlots][kSplitCounters];
 }  // namespace xhip
 
@@ -41,73 +41,80 @@ namespace xhip_host {
 
 namespace {
 constexpr int kMaxDev = 64;
+
+// Which streams own the N slots of one kind on a device.
+template <int N>
+struct Owners {
+    int nused = 0;
+    hipStream_t owner[N] = {};
+    bool released[N] = {};
+
+    // The slot of `st`, now its own if it had none; -1 when other streams own
+    // all of them.
+    int take(hipStream_t st) {
+        int freed = -1;
+        for (int i = 0; i < nused; ++i) {
+            if (!released[i] && owner[i] == st) return i;
+            if (released[i] && freed < 0) freed = i;
+        }
+        if (freed < 0 && nused == N) return -1;
+        const int slot = freed >= 0 ? freed : nused++;
+        owner[slot] = st;
+        released[slot] = false;
+        return slot;
+    }
+    void release(hipStream_t st) {
+        for (int i = 0; i < nused; ++i)
+            if (owner[i] == st && !released[i]) {
+                released[i] = true;
+                owner[i] = nullptr;
+            }
+    }
+};
+
 struct DevSlots {
     bool resolved = false;
     float* partials = nullptr;    // device address of g_splitk_partials on this device
     uint32_t* counters = nullptr; // device address of g_splitk_counters on this device
-    float* sk = nullptr;          // device address of g_sk_partials on this device
-    int nused = 0;
-    hipStream_t owner[xhip::kSplitSlots] = {};
-    bool released[xhip::kSplitSlots] = {};
+    Owners<xhip::kSplitSlots> slots;
+    float* group[xhip::kSkGroups] = {};  // device addresses of the area groups placed so far
+    Owners<xhip::kSkAreas> areas;
 };
 std::mutex g_mu;
 DevSlots g_devs[kMaxDev];
+
+int current_device() {
+    int dev = 0;
+    return hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDev ? dev : -1;
+}
+
+typedef float* (*GroupBase)();
+const GroupBase kGroupBase[xhip::kSkGroups] = {sk_group_base<0>, sk_group_base<1>, sk_group_base<2>,
+                                               sk_group_base<3>, sk_group_base<4>, sk_group_base<5>};
 }  // namespace
 
-namespace {
-
-// The slot of `st` on the current device, whose addresses go to *out; -1 when
-// the device's slots are all owned by other streams or the symbol lookup
-// failed.
-int slot_of(hipStream_t st, DevSlots* out) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return -1;
+// The split-K slot of `st` on the current device: its partials (capacity in
+// floats) and counters (count).  Returns false when the device's slots are
+// all owned by other streams or the symbol lookup failed.
+bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint32_t** counters,
+                 int* ncounters) {
+    const int dev = current_device();
+    if (dev < 0) return false;
     std::lock_guard<std::mutex> lock(g_mu);
     DevSlots& d = g_devs[dev];
     if (!d.resolved) {
         void* pa = nullptr;
         void* ca = nullptr;
-        void* ga = nullptr;
         if (hipGetSymbolAddress(&pa, HIP_SYMBOL(xhip::g_splitk_partials)) != hipSuccess ||
-            hipGetSymbolAddress(&ca, HIP_SYMBOL(xhip::g_splitk_counters)) != hipSuccess ||
-            hipGetSymbolAddress(&ga, HIP_SYMBOL(xhip::g_sk_partials)) != hipSuccess || !pa || !ca || !ga) {
+            hipGetSymbolAddress(&ca, HIP_SYMBOL(xhip::g_splitk_counters)) != hipSuccess || !pa || !ca) {
             (void)hipGetLastError();
-            return -1;
+            return false;
         }
         d.partials = reinterpret_cast<float*>(pa);
         d.counters = reinterpret_cast<uint32_t*>(ca);
-        d.sk = reinterpret_cast<float*>(ga);
         d.resolved = true;
     }
-    int slot = -1, freed = -1;
-    for (int i = 0; i < d.nused; ++i) {
-        if (d.owner[i] == st && !d.released[i]) slot = i;
-        if (d.released[i] && freed < 0) freed = i;
-    }
-    if (slot < 0) {
-        if (freed >= 0) {
-            slot = freed;
-        } else {
-            if (d.nused == xhip::kSplitSlots) return -1;
-            slot = d.nused++;
-        }
-        d.owner[slot] = st;
-        d.released[slot] = false;
-    }
-    out->partials = d.partials;
-    out->counters = d.counters;
-    out->sk = d.sk;
-    return slot;
-}
-
-}  // namespace
-
-// The split-K slot of `st` on the current device: its partials (capacity in
-// floats) and counters (count).  Returns false when there is none.
-bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint32_t** counters,
-                 int* ncounters) {
-    DevSlots d;
-    const int slot = slot_of(st, &d);
+    const int slot = d.slots.take(st);
     if (slot < 0) return false;
     *partials = d.partials + (size_t)slot * xhip::kSplitPartialFloats;
     *partial_floats = xhip::kSplitPartialFloats;
@@ -116,32 +123,32 @@ bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint3
     return true;
 }
 
-// The same slot for the prefill GEMM (gemm_sk_int4.hip): the first
-// kSkSlots slots have 64 MiB for its partial tiles, the others make do with
-// the slot's 4 MiB.
-bool sk_slot(hipStream_t st, float** partials, size_t* partial_floats) {
-    DevSlots d;
-    const int slot = slot_of(st, &d);
-    if (slot < 0) return false;
-    const bool big = slot < xhip::kSkSlots;
-    *partials = big ? d.sk + (size_t)slot * xhip::kSkPartialFloats
-                    : d.partials + (size_t)slot * xhip::kSplitPartialFloats;
-    *partial_floats = big ? xhip::kSkPartialFloats : xhip::kSplitPartialFloats;
-    return true;
-}
-
-// Gives the split-K slot of `st` on the current device back (its counters
-// are zero once the stream's work has finished).
-void splitk_release(hipStream_t st) {
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return;
+// The area of `st` on the current device for the prefill GEMM's partial
+// tiles, kSkAreaFloats floats; null when there is none.
+float* sk_area(hipStream_t st) {
+    const int dev = current_device();
+    if (dev < 0) return nullptr;
     std::lock_guard<std::mutex> lock(g_mu);
     DevSlots& d = g_devs[dev];
-    for (int i = 0; i < d.nused; ++i)
-        if (d.owner[i] == st && !d.released[i]) {
-            d.released[i] = true;
-            d.owner[i] = nullptr;
-        }
+    const int area = d.areas.take(st);
+    if (area < 0) return nullptr;
+    int group = 0, first = 0;
+    while (area >= first + xhip::sk_group_areas(group)) first += xhip::sk_group_areas(group++);
+    if (!d.group[group] && !(d.group[group] = kGroupBase[group]())) {
+        d.areas.release(st);
+        return nullptr;
+    }
+    return d.group[group] + (size_t)(area - first) * xhip::kSkAreaFloats;
+}
+
+// Gives the split-K slot and the area of `st` on the current device back (the
+// slot's counters are zero once the stream's work has finished).
+void splitk_release(hipStream_t st) {
+    const int dev = current_device();
+    if (dev < 0) return;
+    std::lock_guard<std::mutex> lock(g_mu);
+    g_devs[dev].slots.release(st);
+    g_devs[dev].areas.release(st);
 }
 
 }  // namespace xhip_host
