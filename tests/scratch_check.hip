@@ -39,11 +39,12 @@ int main() {
     int areas = 0;
     for (int g = 0; g < xhip::kSkGroups; ++g) areas += xhip::sk_group_areas(g);
     CHECK(areas == xhip::kSkAreas);
-    std::set<float*> seen;
+    std::set<void*> seen;
     float* of[xhip::kSkAreas];
     for (int i = 0; i < xhip::kSkAreas; ++i) {
-        of[i] = sk_area(stream(i));
-        CHECK(of[i] && seen.insert(of[i]).second);
+        const SkArea a = sk_area(stream(i));
+        of[i] = a.part;
+        CHECK(a.part && a.enqueue && seen.insert(a.part).second && seen.insert(a.enqueue).second);
         int placed = 0;
         for (int g = 0; g < xhip::kSkGroups; ++g) {
             CHECK(asked[g] <= 1);
@@ -54,11 +55,11 @@ int main() {
         const size_t at = ((uintptr_t)of[i] & (((uintptr_t)1 << 40) - 1)) / 4;
         CHECK(at % xhip::kSkAreaFloats == 0 && (int)(at / xhip::kSkAreaFloats) < xhip::sk_group_areas(g));
     }
-    for (int i = 0; i < xhip::kSkAreas; ++i) CHECK(sk_area(stream(i)) == of[i]);
-    CHECK(sk_area(stream(50)) == nullptr);
+    for (int i = 0; i < xhip::kSkAreas; ++i) CHECK(sk_area(stream(i)).part == of[i]);
+    CHECK(sk_area(stream(50)).part == nullptr);
     splitk_release(stream(7));
-    CHECK(sk_area(stream(50)) == of[7]);
-    CHECK(sk_area(stream(7)) == nullptr);
+    CHECK(sk_area(stream(50)).part == of[7]);
+    CHECK(sk_area(stream(7)).part == nullptr);
     printf("bad %d\n", bad);
     return bad != 0;
 }

@@ -9,7 +9,7 @@
 namespace xhip_host {
 int num_cus() { return 256; }
 int launch_status() { return 0; }
-float* sk_area(hipStream_t) { return nullptr; }
+SkArea sk_area(hipStream_t) { return {nullptr, nullptr}; }
 int gemm_ws_linear(hipStream_t, void*, const void*, const uint8_t*, const uint16_t*, const float*, int64_t, int64_t,
                    int64_t, bool, int*) { return 1; }
 }

@@ -120,6 +120,39 @@ def test_streams_past_the_areas():
                 assert torch.equal(ys[r, i], solo[j]), (r, i)
 
 
+def test_threads_on_one_stream():
+    """Two host threads with cut calls of different shapes on one stream: each
+    result is what the call gives alone."""
+    import threading
+    import torch
+    from xinfer_amd import ops
+    shapes = [(40, 640, 5120), (300, 136, 2560)]
+    calls = []
+    for M, N, K in shapes:
+        W, S, Xb = _inputs(M, N, K, M)
+        calls.append((M, N, K, to_dev(W), f16_dev(S), f16_dev(Xb), torch.full((30, M, N), float("nan"), device="cuda")))
+    solo = []
+    for M, N, K, dW, dS, dX, ys in calls:
+        solo.append(torch.empty((M, N), device="cuda"))
+        ops.linear_int4(solo[-1], dX, dW, dS, None, M, N, K)
+    stream = torch.cuda.current_stream().cuda_stream
+    torch.cuda.synchronize()
+
+    def work(M, N, K, dW, dS, dX, ys):
+        for y in ys:
+            ops.linear_int4(y, dX, dW, dS, None, M, N, K, stream=stream)
+
+    threads = [threading.Thread(target=work, args=c) for c in calls]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for c, want in zip(calls, solo):
+        for y in c[-1]:
+            assert torch.equal(y, want)
+
+
 def test_graph_replay():
     """A captured gate/up + down pair, replayed with other work in between:
     every replay bit-identical to the eager pass."""

@@ -70,3 +70,18 @@ def test_scratch_owners(tmp_path):
     run = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     print(run.stdout)
     assert run.returncode == 0, run.stdout[-2000:]
+
+
+@pytest.mark.skipif(_hipcc() is None, reason="hipcc not available")
+def test_prefill_gemm_launch_pairs(tmp_path):
+    """The two launches of a cut prefill call, with several host threads on a
+    stream."""
+    exe = str(tmp_path / "sk_enqueue_check")
+    build = subprocess.run([_hipcc(), "-O1", "-std=c++17", "--offload-arch=gfx950",
+                            "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+                            os.path.join(HERE, "sk_enqueue_check.hip"), "-o", exe, "-pthread"],
+                           capture_output=True, text=True, timeout=900)
+    assert build.returncode == 0, build.stderr[-2000:]
+    run = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    print(run.stdout)
+    assert run.returncode == 0, run.stdout[-2000:]

@@ -645,7 +645,6 @@ __global__ __launch_bounds__(256) void gemm_sk_sum_kernel(const SkParams p) {
 using namespace xhip;
 
 namespace xhip_host {
-float* sk_area(hipStream_t st);  // scratch.hip
 int gemm_ws_linear(hipStream_t st, void* Y, const void* X, const uint8_t* W, const uint16_t* S, const float* bias,
                    int64_t M, int64_t N, int64_t K, bool residual, int* rc);  // gemm_ws_int4.hip
 }
@@ -737,11 +736,11 @@ int sk_launch(hipStream_t st, const xinfer_fused_desc* descs, int nd, const uint
     using namespace xhip_host;
     const bool swiglu = W2 != nullptr;
     SkPlan pl = sk_plan(descs, nd, swiglu, M, K, kSkAreaFloats, num_cus());
-    float* part = nullptr;
-    if (!pl.whole && !(part = sk_area(st))) pl = sk_plan(descs, nd, swiglu, M, K, 0, num_cus());
+    SkArea area = {};
+    if (!pl.whole && !(area = sk_area(st)).part) pl = sk_plan(descs, nd, swiglu, M, K, 0, num_cus());
     SkParams p = {};
     p.X = reinterpret_cast<const f16*>(X);
-    p.part = part;
+    p.part = area.part;
     p.M = (int32_t)M;
     p.K = (int32_t)K;
     p.ng = (int32_t)(K / kGroup);
@@ -774,6 +773,9 @@ int sk_launch(hipStream_t st, const xinfer_fused_desc* descs, int nd, const uint
                                 : sk_kernels<false, f16>(pl.mt);
     const int lds = sk::lds_bytes(pl.mt);
     if (!sk_allow_lds(k.main, lds)) return XINFER_ERR_HIP;
+    // the two launches of a cut call stay together on the stream
+    std::unique_lock<std::mutex> together;
+    if (!pl.whole) together = std::unique_lock<std::mutex>(*area.enqueue);
     hipLaunchKernelGGL(k.main, dim3((unsigned)pl.nb), dim3(64 * sk::kWaves), lds, st, p);
     if (int rc = launch_status()) return rc;
     if (pl.whole || (p.r == 0 && p.q % p.ns == 0)) return XINFER_OK;  // every run starts with a tile

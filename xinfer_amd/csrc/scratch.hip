@@ -14,17 +14,17 @@
 // runs on.  A slot belongs to one stream of a device until
 // xinfer_stream_release gives it back: calls on one stream run in order, so
 // they never share a slot concurrently, and calls on different streams use
-// different slots.  Every counter is zero at load time and is returned to
-// zero by the block that finishes its tile range, so a slot needs no
-// clearing between calls.  When every slot of a device is taken (more live
+// different slots.  (A call that uses a slot is one launch, so host threads
+// that share a stream need no more than the stream's own order.)  Every counter
+// is zero at load time and is returned to zero by the block that finishes its
+// tile range, so a slot needs no clearing between calls.  When every slot of a device is taken (more live
 // streams than slots) the caller plans without a cross-block split instead.
 //
 // The prefill GEMM's partial tiles have areas of their own (sk_areas.hip), 64
 // MiB for each stream whose calls leave such tiles, for up to kSkAreas streams
 // of a device, owned and given back as the slots are; with every area owned
-// its calls run as whole tiles.
-
-#include <mutex>
+// its calls run as whole tiles.  Such a call is two launches, which the area's
+// lock keeps together where several host threads enqueue to one stream.
 
 #include "sk_areas.h"
 
@@ -79,6 +79,7 @@ struct DevSlots {
     Owners<xhip::kSplitSlots> slots;
     float* group[xhip::kSkGroups] = {};  // device addresses of the area groups placed so far
     Owners<xhip::kSkAreas> areas;
+    std::mutex enqueue[xhip::kSkAreas];
 };
 std::mutex g_mu;
 DevSlots g_devs[kMaxDev];
@@ -123,22 +124,21 @@ bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint3
     return true;
 }
 
-// The area of `st` on the current device for the prefill GEMM's partial
-// tiles, kSkAreaFloats floats; null when there is none.
-float* sk_area(hipStream_t st) {
+// The area of `st` on the current device for the prefill GEMM's partial tiles.
+SkArea sk_area(hipStream_t st) {
     const int dev = current_device();
-    if (dev < 0) return nullptr;
+    if (dev < 0) return {nullptr, nullptr};
     std::lock_guard<std::mutex> lock(g_mu);
     DevSlots& d = g_devs[dev];
     const int area = d.areas.take(st);
-    if (area < 0) return nullptr;
+    if (area < 0) return {nullptr, nullptr};
     int group = 0, first = 0;
     while (area >= first + xhip::sk_group_areas(group)) first += xhip::sk_group_areas(group++);
     if (!d.group[group] && !(d.group[group] = kGroupBase[group]())) {
         d.areas.release(st);
-        return nullptr;
+        return {nullptr, nullptr};
     }
-    return d.group[group] + (size_t)(area - first) * xhip::kSkAreaFloats;
+    return {d.group[group] + (size_t)(area - first) * xhip::kSkAreaFloats, &d.enqueue[area]};
 }
 
 // Gives the split-K slot and the area of `st` on the current device back (the
