@@ -33,7 +33,8 @@
  * area then; a program that only decodes holds none).  A stream owns its slot
  * and its area, on every device it calls on, until xinfer_stream_release
  * gives them back; with every one owned a call plans without the cross-block
- * split (correct, slower, other rounding of the FP32 sums).  Calls on
+ * split (correct, slower, other rounding of the FP32 sums).
+ * hipStreamPerThread counts as a stream of each calling thread.  Calls on
  * different streams may therefore overlap.  A
  * graph holds the slot and the area of the stream it was captured on: replays
  * of graphs with decode or prefill calls

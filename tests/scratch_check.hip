@@ -2,7 +2,8 @@
 // split-K slots and the prefill GEMM's areas are owned apart, areas of
 // different streams do not overlap, a group of areas is looked up (and thereby
 // placed) only when one of its areas is first asked for, streams past the last
-// area get none, and a released area is handed out again.  Built and run by
+// area get none, a released area is handed out again, and the per-thread
+// stream's handle means another stream on every host thread.  Built and run by
 // tests/test_plan_invariants.py; the runtime's lookups are replaced below.
 #include <hip/hip_runtime.h>
 #define hipGetDevice(p) (*(p) = 0, hipSuccess)
@@ -23,6 +24,7 @@ template <> float* sk_group_base<5>() { return base(5); }
 }
 #include <cstdio>
 #include <set>
+#include <thread>
 using namespace xhip_host;
 static int bad = 0;
 #define CHECK(c) ((c) ? 0 : (printf("FAILED line %d: %s\n", __LINE__, #c), ++bad))
@@ -60,6 +62,22 @@ int main() {
     splitk_release(stream(7));
     CHECK(sk_area(stream(50)).part == of[7]);
     CHECK(sk_area(stream(7)).part == nullptr);
+    for (int i = 0; i < xhip::kSkAreas; ++i) splitk_release(stream(i));
+    for (int i = 100; i < 110; ++i) splitk_release(stream(i));
+    const SkArea here = sk_area(hipStreamPerThread);
+    float* part_here = nullptr;
+    CHECK(splitk_slot(hipStreamPerThread, &part_here, &floats, &cnt, &ncnt));
+    for (int t = 0; t < 2; ++t)
+        std::thread([&] {
+            float* part_there = nullptr;
+            CHECK(splitk_slot(hipStreamPerThread, &part_there, &floats, &cnt, &ncnt) && part_there != part_here);
+            const SkArea there = sk_area(hipStreamPerThread);
+            CHECK(there.part && there.part != here.part && there.enqueue != here.enqueue);
+            CHECK(sk_area(hipStreamPerThread).part == there.part);
+            splitk_release(hipStreamPerThread);  // this thread's, not the other's
+        }).join();
+    CHECK(sk_area(hipStreamPerThread).part == here.part);
+    CHECK(splitk_slot(hipStreamPerThread, &part, &floats, &cnt, &ncnt) && part == part_here);
     printf("bad %d\n", bad);
     return bad != 0;
 }

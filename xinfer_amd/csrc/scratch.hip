@@ -26,6 +26,8 @@
 // its calls run as whole tiles.  Such a call is two launches, which the area's
 // lock keeps together where several host threads enqueue to one stream.
 
+#include <atomic>
+
 #include "sk_areas.h"
 
 namespace xhip {
@@ -42,16 +44,32 @@ namespace xhip_host {
 namespace {
 constexpr int kMaxDev = 64;
 
+// A stream by its handle, and hipStreamPerThread, one handle for a stream of
+// every host thread, by its thread too (numbers are not used again, so a thread
+// that ended without xinfer_stream_release keeps what it owned).
+struct StreamKey {
+    hipStream_t st = nullptr;
+    uint64_t thread = 0;
+    bool operator==(const StreamKey& o) const { return st == o.st && thread == o.thread; }
+};
+
+StreamKey stream_key(hipStream_t st) {
+    if (st != hipStreamPerThread) return {st, 0};
+    static std::atomic<uint64_t> threads{0};
+    thread_local const uint64_t mine = ++threads;
+    return {st, mine};
+}
+
 // Which streams own the N slots of one kind on a device.
 template <int N>
 struct Owners {
     int nused = 0;
-    hipStream_t owner[N] = {};
+    StreamKey owner[N] = {};
     bool released[N] = {};
 
     // The slot of `st`, now its own if it had none; -1 when other streams own
     // all of them.
-    int take(hipStream_t st) {
+    int take(const StreamKey& st) {
         int freed = -1;
         for (int i = 0; i < nused; ++i) {
             if (!released[i] && owner[i] == st) return i;
@@ -63,11 +81,11 @@ struct Owners {
         released[slot] = false;
         return slot;
     }
-    void release(hipStream_t st) {
+    void release(const StreamKey& st) {
         for (int i = 0; i < nused; ++i)
             if (owner[i] == st && !released[i]) {
                 released[i] = true;
-                owner[i] = nullptr;
+                owner[i] = {};
             }
     }
 };
@@ -115,7 +133,7 @@ bool splitk_slot(hipStream_t st, float** partials, size_t* partial_floats, uint3
         d.counters = reinterpret_cast<uint32_t*>(ca);
         d.resolved = true;
     }
-    const int slot = d.slots.take(st);
+    const int slot = d.slots.take(stream_key(st));
     if (slot < 0) return false;
     *partials = d.partials + (size_t)slot * xhip::kSplitPartialFloats;
     *partial_floats = xhip::kSplitPartialFloats;
@@ -130,12 +148,12 @@ SkArea sk_area(hipStream_t st) {
     if (dev < 0) return {nullptr, nullptr};
     std::lock_guard<std::mutex> lock(g_mu);
     DevSlots& d = g_devs[dev];
-    const int area = d.areas.take(st);
+    const int area = d.areas.take(stream_key(st));
     if (area < 0) return {nullptr, nullptr};
     int group = 0, first = 0;
     while (area >= first + xhip::sk_group_areas(group)) first += xhip::sk_group_areas(group++);
     if (!d.group[group] && !(d.group[group] = kGroupBase[group]())) {
-        d.areas.release(st);
+        d.areas.release(stream_key(st));
         return {nullptr, nullptr};
     }
     return {d.group[group] + (size_t)(area - first) * xhip::kSkAreaFloats, &d.enqueue[area]};
@@ -147,8 +165,8 @@ void splitk_release(hipStream_t st) {
     const int dev = current_device();
     if (dev < 0) return;
     std::lock_guard<std::mutex> lock(g_mu);
-    g_devs[dev].slots.release(st);
-    g_devs[dev].areas.release(st);
+    g_devs[dev].slots.release(stream_key(st));
+    g_devs[dev].areas.release(stream_key(st));
 }
 
 }  // namespace xhip_host
