@@ -843,25 +843,13 @@ int mb_swiglu(hipStream_t st, void* Y, const void* X, const uint8_t* Wg, const v
               const uint8_t* Wu, const void* Su, int64_t M, int64_t N, int64_t K,
               int* rc, const float* norm_w = nullptr, float eps = 0.0f);
 int mb_argmax_plan(int64_t M, int64_t N, int64_t K, int* nparts);
-int mb_max_m();  // largest M the small-batch kernel takes (then the GEMM)
+int mb_max_m();  // largest M the small-batch kernel takes
 int mb_argmax(hipStream_t st, float* logits, const void* X, const uint8_t* W, const void* S,
               int64_t M, int64_t N, int64_t K, ArgCand* parts, int* nparts, int* rc);
 int prefill_gemm(hipStream_t st, const xinfer_fused_desc* descs, int nd, const uint8_t* W2, const uint16_t* S2,
                  const void* X, bool y_f32, int64_t M, int64_t K, bool residual);  // gemm_sk_int4.hip
 
-// Whether M rows of K over `rows` weight rows go to the small-batch kernels
-// (true) or to the prefill GEMM.  At M = 9-16 the small-batch kernel stages X
-// at a 16-row stride: where that takes more than two slices of K (K > 5120)
-// and the weights stream for long, the GEMM is faster.  Measured, small-batch
-// -> GEMM: N = 5120, K = 17408, M = 12 / 16 30.0 / 34.5 -> 23.5 / 23.6 us with
-// the residual, N = 10000, K = 9216 27.7 / 30.8 -> 22.3 / 22.4; the other way
-// N = 17408, K = 5120, M = 12 21.3 -> 22.2, norm + gate/up N = 2 x 17408,
-// K = 5120, M = 12 38.8 -> 40.1, N = 2560, K = 9728 13.3 -> 15.8, N = 1024,
-// K = 17408 13.9 -> 17.7.
-bool small_batch(int64_t M, int64_t rows, int64_t K) {
-    if (M < 2 || M > mb_max_m()) return false;
-    return M <= 8 || K <= 5120 || rows * K < 80 * 1000000LL;
-}
+bool small_batch(int64_t M, int64_t rows, int64_t K, bool swiglu);  // gemv_mb_int4.hip; false: the prefill GEMM at M > 8
 }
 
 namespace {
@@ -878,7 +866,7 @@ int linear_f16_impl(void* stream, void* Y, bool y_f32, const void* X, const uint
         !aligned(bias, 4))
         return XINFER_ERR_MISALIGNED;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    if (small_batch(M, N, K)) {
+    if (small_batch(M, N, K, false)) {
         const xinfer_fused_desc one = {Y, W, S, bias, N};
         int mrc = XINFER_OK;
         if (!pairm_linear(st, &one, 1, X, y_f32, M, K, residual, &mrc)) return mrc;
@@ -1007,7 +995,7 @@ int fused_f16_impl(void* stream, const void* X0, const xinfer_fused_desc* descs,
     p.X = reinterpret_cast<const f16*>(X);
     p.norm_w = norm_in_kernel ? norm_w : nullptr;
     p.norm_eps = eps;
-    if (small_batch(M, rows, K)) {
+    if (small_batch(M, rows, K, false)) {
         int mrc = XINFER_OK;
         if (!pairm_linear(st, live, nd, X, false, M, K, false, &mrc)) return mrc;
         if (!mb_linear(st, live, nd, X, false, M, K, false, &mrc)) return mrc;
@@ -1049,7 +1037,7 @@ int swiglu_f16_impl(void* stream, void* Y, const void* X0, const uint8_t* W_gate
     const void* X = X0;
     bool norm_in_kernel = gemv_norm2;  // M = 2: the GEMV's X staging applies the norm
     if (!gemv_norm2 && (rc = norm_input(st, X0, norm_w, eps, M, K, ws, ws_bytes, &X, &norm_in_kernel))) return rc;
-    if (small_batch(M, 2 * N, K) && !gemv_norm2) {
+    if (small_batch(M, 2 * N, K, true) && !gemv_norm2) {
         int mrc = XINFER_OK;
         if (!pairm_swiglu(st, Y, X, W_gate, scales_gate, W_up, scales_up, M, N, K, &mrc)) return mrc;
         if (!mb_swiglu(st, Y, X, W_gate, scales_gate, W_up, scales_up, M, N, K, &mrc))

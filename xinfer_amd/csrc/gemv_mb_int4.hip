@@ -789,11 +789,10 @@ const MbOverrides& mb_overrides() {
 constexpr int64_t kMbWaveSetup = 8;
 
 constexpr size_t kMaxLds = 160 * 1024;
-// Chunked-prefill rows 9..16 fill the 16-row MFMA tile (N = 17408,
-// K = 5120: 21.6 / 25.1 us at M = 9 / 16 against 47 / 48 us for the GEMM,
-// whose 128-row tiles are mostly padding there).  Two to four M-tiles per
-// weight tile (M = 17..64) measured slower than the GEMM: the X slice of
-// 32-64 rows forces 5-10 k-slices and a large split-K combine.
+// Rows 9..16 fill the 16-row MFMA tile (small_batch below has the line to the
+// prefill GEMM there).  Two to four M-tiles per weight tile (M = 17..64)
+// measured slower than a GEMM: the X slice of 32-64 rows forces 5-10 k-slices
+// and a large split-K combine.
 constexpr int kMaxMbM = 16;
 
 }  // namespace
@@ -1155,6 +1154,34 @@ int mb_max_m() {
         return o > 0 ? (o < kMaxMbM ? o : kMaxMbM) : kMaxMbM;
     }();
     return v;
+}
+
+// Whether M rows of K over `rows` weight rows (of both matrices for the
+// SwiGLU) go to the small-batch kernel or to the prefill GEMM.  At M = 9-16
+// the small-batch kernel stages X at a 16-row stride and cuts K > 5120 into
+// slices of up to 16 groups: where the weights stream for long the GEMM is
+// faster, and the sooner the more rows there are.  With K % 2048 == 0 the
+// slices are full and the small-batch SwiGLU holds out longer.  Measured,
+// small-batch -> GEMM, us at M = 9 / 12 / 16 (weights rows * K):
+//   plain   82 M  K = 17408 26.4 / 29.2 / 31 -> 22.9 / 23.0 / 23.5, 6144 21.6 /
+//                 23.1 / 27 -> 21.7 / 21.8 / 22.2; 60 M K = 17408 20.2 / 21.6 /
+//                 24.1 -> 21.0 / 21.0 / 21.1, 12288 17.9 / 18.8 / 20.6 -> 19.6 /
+//                 19.8 / 19.8.  80-105 M at M = 9-10 and K % 2048 == 0 goes
+//                 either way (8192, 92 M 25.3 -> 22.9; 10240, 100 M 22.4 -> 24.5).
+//   SwiGLU  85 M  K = 17408 26.5 / 29.1 / 31.9 -> 25.6 / 26.0 / 25.9, 8192 21.9 /
+//                 23.5 / 25.4 -> 24.3 / 24.5 / 24.7; 100 M K = 12288 23.6 / 26.6
+//                 -> 25.2 / 25.4; 140 M K = 8192 28.9 / 30.9 -> 30.7 / 30.8,
+//                 17408 34.6 / 36.5 -> 30.1 / 30.4; 150 M at M = 10 K = 8192
+//                 30.1 -> 31.6, 14336 33.4 -> 32.1.
+// One slice (K <= 5120): N = 17408, K = 5120 21.2 / 21.9 / 23.2 -> 21.9 / 22.0 /
+// 22.0, K = 2560, 89 M 15.8 / 16.2 / 16.7 -> 22.4 / 22.7 / 22.6; the other way
+// K = 4096, 89 M 23.9 / 25.7 / 28.2 -> 21.8 / 22.0 / 22.1.
+bool small_batch(int64_t M, int64_t rows, int64_t K, bool swiglu) {
+    if (M < 2 || M > mb_max_m()) return false;
+    if (M <= 8 || K <= 5120) return true;
+    int64_t least = 80;
+    if (swiglu && K % 2048 == 0) least = M <= 10 ? 145 : M <= 12 ? 95 : 80;
+    return rows * K < least * 1000000;
 }
 
 int mb_argmax(hipStream_t st, float* logits, const void* X, const uint8_t* W, const void* S,
