@@ -3,7 +3,7 @@
 // every step once, a plan with partial sums fits the scratch slot, the pieces
 // the main kernel leaves are exactly the ones the second launch adds (each
 // split tile once, its pieces in order), and the kernels' float division
-// agrees with integer division.  Built and run by
+// agrees with integer division; and the calls given as arguments are cut.  Built and run by
 // tests/test_plan_invariants.py; no GPU is touched.
 #include "../xinfer_amd/csrc/gemm_sk_int4.hip"
 namespace xhip_host {
@@ -14,6 +14,8 @@ int gemm_ws_linear(hipStream_t, void*, const void*, const uint8_t*, const uint16
                    int64_t, bool, int*) { return 1; }
 }
 #include <cstdio>
+#include <cstdlib>
+#include <cstring>
 #include <map>
 #include <random>
 #include <set>
@@ -28,9 +30,24 @@ static int quotient(int n, int d) {  // sk_div of the kernels
     return q;
 }
 
-int main() {
+// A call whose plan a GPU test relies on, "MT,M,K,swiglu,N[,N..]": cut, with MT
+// row tiles, at least one tile in pieces and one run that starts inside a tile.
+static bool cut_as_said(const char* arg) {
+    int v[8] = {}, n = 0;
+    for (const char* c = arg; c && n < 8; c = strchr(c, ',') ? strchr(c, ',') + 1 : nullptr) v[n++] = atoi(c);
+    xinfer_fused_desc d[4] = {};
+    for (int i = 4; i < n; ++i) d[i - 4].N = v[i];
+    const SkPlan pl = sk_plan(d, n - 4, v[3] != 0, v[1], v[2], xhip::kSkAreaFloats, 256);
+    const int64_t ns = (v[2] / 128 + sk::kwaves(pl.mt) - 1) / sk::kwaves(pl.mt), steps = pl.tiles * pl.mb * ns;
+    const bool ok = n > 4 && !pl.whole && pl.mt == v[0] && (steps % pl.nb || steps / pl.nb % ns);
+    if (!ok) printf("BAD %s: mt %d, runs %d of %lld steps, whole %d\n", arg, pl.mt, pl.nb, (long long)steps, pl.whole);
+    return ok;
+}
+
+int main(int argc, char** argv) {
     std::mt19937_64 rng(2024);
     int bad = 0, whole = 0, cut = 0;
+    for (int i = 1; i < argc; ++i) bad += !cut_as_said(argv[i]);
     for (int it = 0; it < 2000000; ++it) {
         const int d = 1 + (int)(rng() % (rng() % 2 ? 64 : 200000));
         const int n = (int)(rng() % (1 << 24));

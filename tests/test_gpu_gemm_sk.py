@@ -13,6 +13,16 @@ from xinfer_amd import synth
 
 pytestmark = pytest.mark.gpu
 
+# (MT, M, N, K) and (MT, M, Ns, K): calls whose plan has MT row tiles and runs
+# that end inside tiles, so that the second launch adds pieces
+# (tests/test_plan_invariants.py asks the planner for each).  M <= 16: calls
+# that small_batch sends here.
+CUT_SWIGLU = [(1, 23, 200, 8192), (2, 64, 2000, 3456), (3, 96, 4000, 2176), (4, 250, 1500, 2176), (1, 12, 2400, 17408),
+              (1, 13, 6500, 6272)]
+CUT_FUSED = [(1, 23, (300, 48, 130), 5120), (2, 60, (4000, 700, 48), 3456), (3, 90, (4600, 1, 900, 48), 3200),
+             (4, 250, (3000, 1, 300, 48), 2176), (1, 16, (9000, 100), 9088)]
+CUT_GRAPH = [(1, 20, 2048, 3072), (1, 20, 3072, 2048), (3, 300, 136, 2560)]  # gate/up, down, other work
+
 
 @pytest.fixture(scope="module", autouse=True)
 def _gpu():
@@ -77,6 +87,92 @@ def test_swiglu(M, N, K):
     y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
     ops.mlp_gate_up_swiglu_int4(y, f16_dev(Xb), to_dev(W), f16_dev(S), to_dev(U), f16_dev(T), M, N, K)
     _check16(y, oracle.swiglu_int4(oracle.f16_to_f32(Xb), W, S, U, T, M, N, K, nthreads=cpu_threads()))
+
+
+def _cols(N, seed):
+    """Columns that stand for a wide output: both ends and a hundred others."""
+    c = np.random.default_rng(seed).integers(0, N, 100)
+    return np.unique(np.concatenate([c, np.arange(min(N, 40)), np.arange(max(0, N - 40), N)]))
+
+
+@pytest.mark.parametrize("mt,M,N,K", CUT_SWIGLU)
+def test_swiglu_in_pieces(mt, M, N, K):
+    """Also with the norm before it: the bits of norm and SwiGLU called apart."""
+    import torch
+    from xinfer_amd import ops
+    print("case swiglu in pieces", M, N, K, flush=True)
+    W, S = synth.packed_weights(M + N, N, K), synth.scales(M + N, N, K, 0.01)  # keeps SiLU(g) * u near 1 at long K
+    U, T, Xb = synth.packed_weights(M, N, K), synth.scales(M, N, K, 0.01), synth.activations(M + N, M, K)
+    g, u, x = (to_dev(W), f16_dev(S)), (to_dev(U), f16_dev(T)), f16_dev(Xb)
+    y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+    ops.mlp_gate_up_swiglu_int4(y, x, *g, *u, M, N, K)
+    assert torch.isfinite(y).all()
+    c = _cols(N, M)
+    ref = oracle.swiglu_int4(oracle.f16_to_f32(Xb), W[c], S[c], U[c], T[c], M, len(c), K, nthreads=cpu_threads())
+    _check16(y[:, torch.from_numpy(c).cuda()], ref)
+    nw = to_dev(np.random.default_rng(M).normal(1, 0.1, K).astype(np.float32))
+    xn, a, b = torch.empty_like(x), torch.empty_like(y), torch.full_like(y, float("nan"))
+    ops.rmsnorm(xn, x, nw, M, K, 1e-6)
+    ops.mlp_gate_up_swiglu_int4(a, xn, *g, *u, M, N, K)
+    ops.rmsnorm_mlp_gate_up_swiglu_int4(b, x, nw, 1e-6, *g, *u, M, N, K)
+    assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("mt,M,Ns,K", CUT_FUSED)
+def test_fused_with_bias_in_pieces(mt, M, Ns, K):
+    import torch
+    from xinfer_amd import ops
+    print("case fused in pieces", M, Ns, K, flush=True)
+    Xb = synth.activations(M, M, K)
+    x = f16_dev(Xb)
+    descs, refs = [], []
+    for i, N in enumerate(Ns):
+        W, S = synth.packed_weights(M + i, N, K), synth.scales(M + i, N, K)
+        bias = np.linspace(-1 - i, 1, N).astype(np.float32)
+        y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+        descs.append(ops.FusedProjectionDesc(y, to_dev(W), f16_dev(S), to_dev(bias), N))
+        c = _cols(N, i)
+        refs.append((c, oracle.linear_int4(oracle.f16_to_f32(Xb), W[c], S[c], M, len(c), K, nthreads=cpu_threads()) + bias[c]))
+    ops.linear_int4_fused(x, descs, len(Ns), M, K)
+    for d, (c, ref) in zip(descs, refs):
+        assert torch.isfinite(d.Y).all()
+        _check16(d.Y[:, torch.from_numpy(c).cuda()], ref)
+    nw = to_dev(np.random.default_rng(M).normal(1, 0.1, K).astype(np.float32))
+    xn = torch.empty_like(x)
+    ops.rmsnorm(xn, x, nw, M, K, 1e-6)
+    ops.linear_int4_fused(xn, descs, len(Ns), M, K)
+    want = [d.Y.clone() for d in descs]
+    for d in descs:
+        d.Y.fill_(float("nan"))
+    ops.rmsnorm_linear_int4_fused(x, nw, 1e-6, descs, len(Ns), M, K)
+    for d, w in zip(descs, want):
+        assert torch.equal(d.Y, w)
+
+
+def test_more_rows_than_a_slab():
+    """65536 rows go out in one slab, the 17 after them in another."""
+    import torch
+    from xinfer_amd import ops
+    M, Ns, K = 65536 + 17, (16, 40), 128
+    Xb = synth.activations(3, M, K)
+    x, X = f16_dev(Xb), oracle.f16_to_f32(Xb)
+    descs, refs = [], []
+    for N in Ns:
+        W, S = synth.packed_weights(N, N, K), synth.scales(N, N, K)
+        y = torch.full((M, N), float("nan"), dtype=torch.float16, device="cuda")
+        descs.append(ops.FusedProjectionDesc(y, to_dev(W), f16_dev(S), None, N))
+        refs.append(oracle.linear_int4(X, W, S, M, N, K, nthreads=cpu_threads()))
+    ops.linear_int4_fused(x, descs, 2, M, K)
+    for d, ref in zip(descs, refs):
+        _check16(d.Y, ref)
+    d = descs[0]
+    y32 = torch.full((M, d.N), float("nan"), device="cuda")
+    ops.linear_int4(y32, x, d.W_int4, d.scales, None, M, d.N, K)
+    assert np.abs(to_np(y32) - refs[0]).max() <= 1e-4
+    r0 = torch.from_numpy(np.random.default_rng(1).normal(0, 1, (M, d.N))).half().cuda()
+    r = r0.clone()
+    ops.linear_int4_residual(r, x, d.W_int4, d.scales, None, M, d.N, K)
+    assert torch.equal(r, (d.Y.float() + r0.float()).half())
 
 
 def test_streams_past_the_areas():
@@ -154,34 +250,47 @@ def test_threads_on_one_stream():
 
 
 def test_graph_replay():
-    """A captured gate/up + down pair, replayed with other work in between:
-    every replay bit-identical to the eager pass."""
+    """A captured gate/up + down pair, both in pieces, replayed on its stream
+    with other X each time and another call in pieces between the replays:
+    every result bit-identical to the eager pass on another stream."""
     import torch
     from xinfer_amd import ops
-    M, N, K = 50, 1024, 1536
-    W, S, Xb = _inputs(M, N, K, 9)
+    (_, M, N, K), (_, _, N2, K2), (_, m, n, k) = CUT_GRAPH
+    assert (N2, K2) == (K, N)
+    W, S, _ = _inputs(M, N, K, 9)
     U, T, _ = _inputs(M, N, K, 10)
     D, E, _ = _inputs(M, K, N, 11)
-    g, u, d = (to_dev(W), f16_dev(S)), (to_dev(U), f16_dev(T)), (to_dev(D), f16_dev(E))
-    x = f16_dev(Xb)
+    O, P, Zb = _inputs(m, n, k, 12)
+    g, u, d, o = (to_dev(W), f16_dev(S)), (to_dev(U), f16_dev(T)), (to_dev(D), f16_dev(E)), (to_dev(O), f16_dev(P))
+    xs, z = [f16_dev(synth.activations(20 + i, M, K)) for i in range(5)], f16_dev(Zb)
+    x = torch.empty_like(xs[0])
     act = torch.empty((M, N), dtype=torch.float16, device="cuda")
     out = torch.empty((M, K), dtype=torch.float16, device="cuda")
+    other, want_other = torch.empty((m, n), device="cuda"), torch.empty((m, n), device="cuda")
 
     def step():
         ops.mlp_gate_up_swiglu_int4(act, x, *g, *u, M, N, K)
         ops.linear_int4(out, act, *d, None, M, K, N)
 
-    step()
+    want = []
+    for xi in xs:
+        x.copy_(xi)
+        step()
+        want.append((act.clone(), out.clone()))
+    ops.linear_int4(want_other, z, *o, None, m, n, k)
     torch.cuda.synchronize()
-    want = out.clone()
+    stream = torch.cuda.Stream()
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph):
+    with torch.cuda.graph(graph, stream=stream):
         step()
-    for _ in range(4):
-        out.zero_()
-        act.zero_()
-        graph.replay()
-        torch.cuda.synchronize()
-        assert torch.equal(out, want)
-        step()
-        torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        for xi, (wa, wo) in zip(xs, want):
+            x.copy_(xi)
+            out.zero_()
+            act.zero_()
+            other.zero_()
+            ops.linear_int4(other, z, *o, None, m, n, k)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(act, wa) and torch.equal(out, wo)
+            assert torch.equal(other, want_other)

@@ -46,14 +46,19 @@ def test_pair_split(tmp_path):
 @pytest.mark.skipif(_hipcc() is None, reason="hipcc not available")
 def test_prefill_gemm_split(tmp_path):
     """The prefill GEMM's work split: runs, pieces and the second launch that
-    adds them, over 20000 random calls."""
+    adds them, over 20000 random calls; and the calls that the GPU tests make
+    for the sake of their pieces are cut."""
+    from tests.test_gpu_gemm_sk import CUT_FUSED, CUT_GRAPH, CUT_SWIGLU
+    calls = [(mt, M, K, 0, *Ns) for mt, M, Ns, K in CUT_FUSED]
+    calls += [(mt, M, K, 1, N) for mt, M, N, K in CUT_SWIGLU + CUT_GRAPH[:1]]
+    calls += [(mt, M, K, 0, N) for mt, M, N, K in CUT_GRAPH[1:]]
     exe = str(tmp_path / "sk_plan_check")
     build = subprocess.run([_hipcc(), "-O1", "-std=c++17", "--offload-arch=gfx950",
                             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
                             os.path.join(HERE, "sk_plan_check.hip"), "-o", exe],
                            capture_output=True, text=True, timeout=900)
     assert build.returncode == 0, build.stderr[-2000:]
-    run = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    run = subprocess.run([exe, *(",".join(map(str, c)) for c in calls)], capture_output=True, text=True, timeout=300)
     print(run.stdout)
     assert run.returncode == 0, run.stdout[-2000:]
 

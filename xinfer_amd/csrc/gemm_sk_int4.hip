@@ -396,7 +396,7 @@ __global__ __launch_bounds__(64 * sk::kWaves) void gemm_sk_int4_kernel(const SkP
             const unsigned char* xs = smem + xat;
             f32x16 pa[P0], pb[P1 > 0 ? P1 : 1];
             constexpr int CPK = P1 > 0 ? 1 : 2;  // copies per 16-k step
-            static_assert(CPW <= (P1 > 0 ? 8 : 8), "copies before the middle");
+            static_assert(CPW <= (P1 > 0 ? 8 : 4) * CPK, "copies before the middle");
             b[0] = sk_decode8(w[0][0]);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
