@@ -4,7 +4,8 @@
 
 (1) runs in a fresh child process: the library is loaded and its first call
 ever -- a small-batch projection that splits K over blocks (M = 4,
-K = 17408, N = 5120, the down projection of config 2) -- is made inside
+K = 17408, N = 5120, the down projection of config 2), or a prefill one that
+leaves partial tiles, whose area is placed then -- is made inside
 torch.cuda.graph capture (capture_error_mode "global": any allocation or
 device synchronisation inside the call fails the capture).  Replays are
 compared with the oracle.
@@ -25,6 +26,7 @@ import pytest
 import oracle
 from tests import kat
 from tests.gpu_util import cpu_threads, f16_dev, to_dev, to_np
+from tests.test_gpu_gemm_sk import CUT_STREAMS
 from xinfer_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -50,7 +52,7 @@ import sys, numpy as np, torch
 sys.path.insert(0, sys.argv[1])
 import oracle
 from xinfer_amd import synth, ops
-M, N, K = 4, 5120, 17408
+M, N, K = map(int, sys.argv[2:5])
 W, S, Xb = synth.packed_weights(5, N, K), synth.scales(5, N, K), synth.activations(5, M, K)
 dev = torch.device("cuda:0")
 dW = torch.from_numpy(W).to(dev)
@@ -81,9 +83,10 @@ print("first-call capture ok", err)
 """
 
 
-def test_first_call_captured_in_fresh_process():
-    print("case first-call capture M=4 N=5120 K=17408", flush=True)
-    r = subprocess.run([sys.executable, "-c", _CHILD, ROOT], capture_output=True, text=True,
+@pytest.mark.parametrize("M,N,K", [(4, 5120, 17408), CUT_STREAMS[1][1:]])
+def test_first_call_captured_in_fresh_process(M, N, K):
+    print("case first-call capture", M, N, K, flush=True)
+    r = subprocess.run([sys.executable, "-c", _CHILD, ROOT, str(M), str(N), str(K)], capture_output=True, text=True,
                        timeout=300, cwd=ROOT)
     print(r.stdout[-2000:], r.stderr[-3000:])
     assert r.returncode == 0, r.stderr[-3000:]

@@ -21,6 +21,7 @@ CUT_SWIGLU = [(1, 23, 200, 8192), (2, 64, 2000, 3456), (3, 96, 4000, 2176), (4, 
               (1, 13, 6500, 6272)]
 CUT_FUSED = [(1, 23, (300, 48, 130), 5120), (2, 60, (4000, 700, 48), 3456), (3, 90, (4600, 1, 900, 48), 3200),
              (4, 250, (3000, 1, 300, 48), 2176), (1, 16, (9000, 100), 9088)]
+CUT_STREAMS = [(4, 512, 136, 640), (1, 40, 640, 5120), (3, 300, 136, 2560)]  # many streams; two threads; a first call
 CUT_GRAPH = [(1, 20, 2048, 3072), (1, 20, 3072, 2048), (3, 300, 136, 2560)]  # gate/up, down, other work
 
 
@@ -183,7 +184,7 @@ def test_streams_past_the_areas():
     import ctypes
     import torch
     from xinfer_amd import _lib, ops
-    M, N, K = 512, 136, 640  # 20 runs over 4 tiles; 4 runs of whole tiles without an area
+    _, M, N, K = CUT_STREAMS[0]  # whole tiles without an area
     W, S, _ = _inputs(M, N, K, 5)
     Xs = [synth.activations(100 + i, M, K) for i in range(36)]
     dW, dS, dXs = to_dev(W), f16_dev(S), [f16_dev(x) for x in Xs]
@@ -222,9 +223,8 @@ def test_threads_on_one_stream():
     import threading
     import torch
     from xinfer_amd import ops
-    shapes = [(40, 640, 5120), (300, 136, 2560)]
     calls = []
-    for M, N, K in shapes:
+    for _, M, N, K in CUT_STREAMS[1:]:
         W, S, Xb = _inputs(M, N, K, M)
         calls.append((M, N, K, to_dev(W), f16_dev(S), f16_dev(Xb), torch.full((30, M, N), float("nan"), device="cuda")))
     solo = []

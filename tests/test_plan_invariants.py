@@ -48,10 +48,10 @@ def test_prefill_gemm_split(tmp_path):
     """The prefill GEMM's work split: runs, pieces and the second launch that
     adds them, over 20000 random calls; and the calls that the GPU tests make
     for the sake of their pieces are cut."""
-    from tests.test_gpu_gemm_sk import CUT_FUSED, CUT_GRAPH, CUT_SWIGLU
+    from tests.test_gpu_gemm_sk import CUT_FUSED, CUT_GRAPH, CUT_STREAMS, CUT_SWIGLU
     calls = [(mt, M, K, 0, *Ns) for mt, M, Ns, K in CUT_FUSED]
     calls += [(mt, M, K, 1, N) for mt, M, N, K in CUT_SWIGLU + CUT_GRAPH[:1]]
-    calls += [(mt, M, K, 0, N) for mt, M, N, K in CUT_GRAPH[1:]]
+    calls += [(mt, M, K, 0, N) for mt, M, N, K in CUT_GRAPH[1:] + CUT_STREAMS]
     exe = str(tmp_path / "sk_plan_check")
     build = subprocess.run([_hipcc(), "-O1", "-std=c++17", "--offload-arch=gfx950",
                             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
