@@ -75,7 +75,8 @@ const char* xinfer_status_string(int status);
  * DeviceContext and never destroyed).  For long-running callers that create
  * and destroy streams: waits for `stream`'s work, then gives back its
  * split-K slot and its area for partial tiles and frees its argmax scratch on
- * the current device, so a later stream can take them.  Call it before
+ * the current device, so a later stream can take them (graphs captured on
+ * `stream` must not be replayed after that).  Call it before
  * hipStreamDestroy; without it a destroyed stream keeps its slot and area until
  * the process ends. */
 int xinfer_stream_release(void* stream);
@@ -86,13 +87,14 @@ const char* xinfer_version(void);
 /* ---------------------------------------------------------------------------
  * linear_int4: Y[m][n] = sum_g fp32(S[n][g]) * sum_{j<128} X[m][128g+j] *
  *              q[n][128g+j] (+ bias[n]), FP32 accumulation.
- * M <= 16 runs the bandwidth-bound decode kernels (VALU GEMV at M = 1-2,
- * MFMA small-batch kernel at M = 2-16); larger M (chunked prefill) runs the
- * MFMA GEMM, as the reference routes both through this one call
+ * M <= 8 runs the bandwidth-bound decode kernels (VALU GEMV at M = 1-2,
+ * MFMA small-batch kernel at M = 2-8); larger M (chunked prefill) runs the
+ * MFMA GEMM, or up to M = 16 the small-batch kernel where K <= 5120 or the
+ * weights are few, as the reference routes all through this one call
  * (src/targets/qwen3_8/forward.cpp:284-287).  Dequantisation: every kernel
  * multiplies the exact integer q by the FP32 group scale, as the reference
- * does, but for one: fp16 outputs of launches that fill the chip with 256-row
- * blocks feed the matrix cores B = fp16(q*s), rounded once per weight
+ * does, but for one: fp16 outputs of one projection whose 256-row blocks fill
+ * the chip feed the matrix cores B = fp16(q*s), rounded once per weight
  * (relative error <= 2^-11, inside the fp16 output's rounding).
  * ------------------------------------------------------------------------- */
 

@@ -1,4 +1,5 @@
-// INT4-G128-SYM projection GEMM for prefill rows (M > 16) on gfx950:
+// INT4-G128-SYM projection GEMM for prefill rows on gfx950 (M > 16, and M =
+// 9-16 where small_batch() of gemv_mb_int4.hip sends many weights here):
 // weights decoded in registers, work split evenly over the CUs.
 //
 // Same contract as the reference's linear_int4 / linear_int4_fused /
@@ -18,16 +19,20 @@
 // of a tile, e.g. 13 x 128 KB for N = 5120, K = 17408, M = 128: 74.0 against
 // 41.2 us.)
 //
-// What bounds it: at M <= 64 the weights' arrival and the decode (12 VALU per
-// packed dword, two waves per SIMD), at larger M the MFMAs at the clock that
-// they leave (1.46 GHz at M = 128, N = 69632, matrix cores busy 53 %).
-// N = 17408, K = 5120, M = 17 / 64 / 128: 21.9 / 26.7 / 40.8 us = 2.0 / 1.7 /
-// 1.1 TB/s of weights, 138 / 427 / 559 TFLOP/s (the 128-row GEMM with a block
+// What bounds it (N = 69632, K = 5120, test builds without a part; M = 32 / 64 /
+// 96 / 128, full 58.7 / 75.5 / 89.8 / 109.5 us): up to M = 64 the copies to LDS
+// and the barriers between them (55.3 / 67.6 us without MFMA and decode), at
+// larger M these (73.9 / 88.8) and the rest (without copies 72.6 / 90.6) take
+// about four fifths of the time each and overlap only in part; the decode is
+// hidden (111.8 at M = 128 without it), the matrix cores are busy 55 % of the
+// M = 128 launch.
+// N = 17408, K = 5120, M = 17 / 64 / 128: 21.7 / 26.4 / 39.9 us = 2.1 / 1.7 /
+// 1.1 TB/s of weights, 140 / 432 / 572 TFLOP/s (the 128-row GEMM with a block
 // per tile and rounded weights that it replaced: 49.3 / 55.0 / 68.2);
-// N = 5120, K = 17408, M = 23 / 512: 23.2 / 104 us (157 / 201); K = 3456,
-// N = 5003, M = 200, fp32 outputs: 27.0 us (214 as GEMV slabs of 8 rows).
-// Before the run cut, those long-K,
-// small-N shapes left two thirds of the CUs without a block.
+// N = 5120, K = 17408, M = 23 / 512: 23.2 / 107 us (157 / 201); K = 3456,
+// N = 5003, M = 200, fp32 outputs: 27.1 us (214 as GEMV slabs of 8 rows).
+// Before the run cut, those long-K, small-N shapes left two thirds of the CUs
+// without a block.
 
 #include <stdlib.h>
 
@@ -694,13 +699,18 @@ int64_t sk_tiles(const xinfer_fused_desc* descs, int nd, bool swiglu, int mt) {
     return tiles;
 }
 
-// Smallest estimated time, in us.  Measured on MI355X: a step of MT row tiles
-// takes kStep[MT][0] with few blocks running and kStep[MT][1] with one on
-// every CU (they share HBM, L2 and power); start, first loads and stores 5.5;
-// the second launch 3 and 0.35 per piece of a tile.  E.g. N = 1024, K = 5120,
-// M = 128 (160 steps): 80 runs 21.6, 32 runs 18.5, 16 runs 23.1 us; N = 3000,
-// K = 1024, M = 64: runs of whole tiles 9.2, 96 runs 10.2 us; N = 17408,
-// K = 5120, M = 17 / 64: 256 runs 21.6 / 27.3, whole tiles 23.7 / 32.5 us.
+// Smallest estimated time, in us: a step of MT row tiles takes kStep[MT][0]
+// with few blocks running and kStep[MT][1] with one on every CU (they share
+// HBM, L2 and power); start, first loads and stores 5.5; the second launch 3
+// and 0.35 per piece of a tile.  kStep is from before a step's first operands
+// were read ahead and the LDS order changed; with a block on every CU a step
+// now takes 1.10 / 1.46 / 1.70 / 2.06 at MT = 1 .. 4.  A piece is counted alike
+// at 16 KB (MT = 1) and 128 KB (MT = 4): sums of N = 5003, K = 3456, M = 200
+// take 9.2 us where 5.2 are estimated, of {10240, 6144, 48, 48} x 5120, M = 77
+// 7.2 where 4.6.  Measured, chosen plan first: N = 1024, K = 5120, M = 128 14.8,
+// 32 runs 18.3, 16 runs 25.5; N = 3000, K = 1024, M = 64 whole tiles 8.0, 96
+// runs 10.7; N = 17408, K = 5120, M = 17 / 64 256 runs 21.6 / 26.4, whole tiles
+// 23.3 / 29.8.
 SkPlan sk_plan(const xinfer_fused_desc* descs, int nd, bool swiglu, int64_t M, int64_t K, size_t part_floats, int cus) {
     static const double kStep[5][2] = {{0, 0}, {0.8, 1.1}, {1.0, 1.5}, {1.2, 1.85}, {1.45, 2.2}};
     const int64_t ng = K / kGroup, rows = (M + 31) / 32;

@@ -832,7 +832,7 @@ int gemv_f16(hipStream_t st, const GemvParams& base, int64_t M) {
 }  // namespace xhip_host
 
 // Forward declarations: M > 8 with fp16 activations (chunked prefill) and
-// the MFMA small-batch kernel for 2 <= M <= 8 (gemv_mb_int4.hip; each returns
+// the MFMA small-batch kernel for 2 <= M <= 16 (gemv_mb_int4.hip; each returns
 // 1 when the shape is left to the VALU GEMV here).
 namespace xhip_host {
 // norm_w: RMSNorm of X inside the kernel (M = 3, 4, 8 with every row whole in

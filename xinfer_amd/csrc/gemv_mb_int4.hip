@@ -1,4 +1,4 @@
-// INT4-G128-SYM small-batch decode projection (2 <= M <= 8) on gfx950.
+// INT4-G128-SYM small-batch decode projection (2 <= M <= 16) on gfx950.
 //
 // Same contract as the reference's sub-group GEMV at M > 1 (the batched rows
 // of src/ops/linear.cpp:165-305, the fused variants 351-498 and 501-617, and
